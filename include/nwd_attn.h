@@ -316,7 +316,10 @@ enum {
 /* matmul_nbits_sg.wgsl main (:81-137) for `batch` activation rows:
  * y[b][n] = epilogue(W . a[b]). a is [batch][32 * n_blocks] f32 (16-byte
  * aligned), y [batch][n] f32. Dispatched as ceil(N / 4) workgroups by the
- * reference (engine/runtime.js:359-361); here the library picks the grid. */
+ * reference (engine/runtime.js:359-361); here the library picks the grid.
+ * Calls of several rows (and nwd_qkv_append's, nwd_lm_head_argmax's) past a
+ * size run on fp16 MFMAs, the activations carried as high and low parts in
+ * the context's workspace: closer to 64 bits than the one-row kernels. */
 int nwd_q4_gemv(nwd_ctx* ctx, const float* a, const nwd_q4_weight* w, float* y,
                 int32_t batch, int32_t epilogue, void* stream);
 

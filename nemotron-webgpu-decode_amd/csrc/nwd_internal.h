@@ -165,9 +165,39 @@ constexpr int kQ4MaxBlocks = 256;
 
 enum Q4Epilogue { kQ4None = 0, kQ4Relu2 = 1, kQ4Accumulate = 2 };
 
+// Workspace that a projection of several rows converts its activations into
+// (nwd_q4_rows.hip): 16-byte aligned device memory of the context.
+struct Q4Scratch {
+  void* base;
+  size_t bytes;
+};
+
+// Whether the matrix-core kernels take a projection of n columns (all three
+// for q/k/v, `narrowest` the fewest of them) and `rows` rows; pick: with the
+// greedy pick. Below the products of rows and 32-weight cells here the
+// one-row kernels are faster, whose one launch and 2-5 us per million cells
+// and row stand against two launches (us per call, one-row against matrix-
+// core, K and columns as given: 3136 x 7168, 2 and 3 rows 10.5 against 11.0
+// and 14.8 against 11.2; 5120 x 3136, 2 and 3 rows 9.0 against 10.1 and 11.8
+// against 10.3; 3136 x 1024, 8 rows 6.6 against 8.3; 896 x 896, 32 and 100
+// rows 8.0 against 7.8 and 20.4 against 9.9; with the pick, 1024 x 40000, 4
+// rows 22.9 against 24.3, 3136 x 131072, 2 rows 94 against 87). The others
+// are what their reads need: 16 cells (one 8-byte run of zero points), byte
+// offsets below 2^31, and scratch for at least 8 rows.
+bool q4_rows_shape(int n, int narrowest, int n_blocks, int rows, bool pick, Q4Scratch scratch);
+hipError_t launch_q4_rows_gemv(const float* x, const Q4Mat& w, int n_blocks, float* y, int rows,
+                               int epilogue, Q4Scratch scratch, hipStream_t stream);
+hipError_t launch_q4_rows_qkv(const Shape& s, const float* x, const Q4Mat& wq, const Q4Mat& wk,
+                              const Q4Mat& wv, int n_blocks, void* q_out, void* k_cache,
+                              void* v_cache, const int32_t* pos, int batch, int* status,
+                              Q4Scratch scratch, hipStream_t stream);
+hipError_t launch_q4_rows_argmax(const float* x, const Q4Mat& w, int n_blocks, float* logits,
+                                 uint32_t* out, int batch, unsigned long long* records,
+                                 Q4Scratch scratch, hipStream_t stream);
+
 // y[b][n] = epilogue(dequant(W) . x[b]) for b < batch; x [batch][K] f32.
 hipError_t launch_q4_gemv(const float* x, const Q4Mat& w, int n_blocks, float* y, int batch,
-                          int epilogue, hipStream_t stream);
+                          int epilogue, Q4Scratch scratch, hipStream_t stream);
 
 // The attention layer's q/k/v projections of x [batch][K] with the new K/V
 // rows rounded to fp16 straight into the caches at pos[b] (q to q_out,
@@ -175,7 +205,7 @@ hipError_t launch_q4_gemv(const float* x, const Q4Mat& w, int n_blocks, float* y
 hipError_t launch_qkv_append(const Shape& s, const float* x, const Q4Mat& wq, const Q4Mat& wk,
                              const Q4Mat& wv, int n_blocks, void* q_out, void* k_cache,
                              void* v_cache, const int32_t* pos, int batch, int* status,
-                             hipStream_t stream);
+                             Q4Scratch scratch, hipStream_t stream);
 
 // The greedy pick of kernels/argmax_partial.wgsl + argmax_merge.wgsl over
 // x [batch][n]: one 64-bit record per chunk of logits in `records`, then a
@@ -194,6 +224,6 @@ hipError_t launch_argmax_merge(const unsigned long long* records, int per_row, i
 int q4_argmax_records_per_row(int n);
 hipError_t launch_q4_argmax(const float* x, const Q4Mat& w, int n_blocks, float* logits,
                             uint32_t* out, int batch, unsigned long long* records,
-                            hipStream_t stream);
+                            Q4Scratch scratch, hipStream_t stream);
 
 }  // namespace nwd

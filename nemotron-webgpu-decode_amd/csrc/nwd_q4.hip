@@ -34,6 +34,10 @@
 // order is not reproduced: results agree with it to float32 rounding (the
 // parity tests bound the difference by 1e-6 of sum |w x|).
 //
+// Calls of several activation rows take the matrix-core kernels of
+// nwd_q4_rows.hip from a size on (q4_rows_shape); here every row streams the
+// weights again.
+//
 // Weight traffic is the roofline: 16.5 bytes per 32 weights (quant, scale,
 // zero point). The activation (12.5 KB at K = 3136) is read by every
 // wavefront from L2.
@@ -545,7 +549,9 @@ hipError_t launch_gemv_split(const float* x, const Q4Mat& w, int n_blocks, float
 }  // namespace
 
 hipError_t launch_q4_gemv(const float* x, const Q4Mat& w, int n_blocks, float* y, int batch,
-                          int epilogue, hipStream_t stream) {
+                          int epilogue, Q4Scratch scratch, hipStream_t stream) {
+  if (q4_rows_shape(w.n, w.n, n_blocks, batch, false, scratch))
+    return launch_q4_rows_gemv(x, w, n_blocks, y, batch, epilogue, scratch, stream);
   switch (q4_split(n_blocks)) {
     case 1: return launch_gemv_split<1>(x, w, n_blocks, y, batch, epilogue, stream);
     case 2: return launch_gemv_split<2>(x, w, n_blocks, y, batch, epilogue, stream);
@@ -557,7 +563,9 @@ int q4_argmax_records_per_row(int n) { return (n + kQ4WgCols - 1) / kQ4WgCols; }
 
 hipError_t launch_q4_argmax(const float* x, const Q4Mat& w, int n_blocks, float* logits,
                             uint32_t* out, int batch, unsigned long long* records,
-                            hipStream_t stream) {
+                            Q4Scratch scratch, hipStream_t stream) {
+  if (q4_rows_shape(w.n, w.n, n_blocks, batch, true, scratch))
+    return launch_q4_rows_argmax(x, w, n_blocks, logits, out, batch, records, scratch, stream);
   const int per_row = q4_argmax_records_per_row(w.n);
   const dim3 grid(per_row, batch);
   const int iters = q4w_iters(n_blocks);  // 0 past 24 blocks per lane (K > 6144)
@@ -592,7 +600,10 @@ hipError_t launch_q4_argmax(const float* x, const Q4Mat& w, int n_blocks, float*
 hipError_t launch_qkv_append(const Shape& s, const float* x, const Q4Mat& wq, const Q4Mat& wk,
                              const Q4Mat& wv, int n_blocks, void* q_out, void* k_cache,
                              void* v_cache, const int32_t* pos, int batch, int* status,
-                             hipStream_t stream) {
+                             Q4Scratch scratch, hipStream_t stream) {
+  if (q4_rows_shape(wq.n + wk.n + wv.n, wk.n < wq.n ? wk.n : wq.n, n_blocks, batch, false, scratch))
+    return launch_q4_rows_qkv(s, x, wq, wk, wv, n_blocks, q_out, k_cache, v_cache, pos, batch,
+                              status, scratch, stream);
   switch (q4_split(n_blocks)) {
     case 1: return launch_qkv_split<1>(s, x, wq, wk, wv, n_blocks, q_out, k_cache, v_cache, pos, batch, status, stream);
     case 2: return launch_qkv_split<2>(s, x, wq, wk, wv, n_blocks, q_out, k_cache, v_cache, pos, batch, status, stream);

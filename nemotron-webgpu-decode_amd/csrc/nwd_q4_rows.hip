@@ -1,0 +1,591 @@
+// nwd_q4_rows.hip — the 4-bit projections of several activation rows at once
+// on the matrix cores (gfx950).
+//
+// nwd_q4.hip runs one workgroup column per activation row: every row streams
+// and unpacks all the weights again. Here a weight is read and unpacked once
+// for up to 64 rows, as the B operand of v_mfma_f32_16x16x32_f16 (one 32-
+// weight block along K is one MFMA's depth):
+//   B  the exact integers nib - zp of one block of 16 columns, in fp16;
+//   A  16 activation rows, each scaled by a power of two so that its largest
+//      magnitude lies in [2^14, 2^15) and carried as fp16 high and low parts
+//      (hi = fp16(x), lo = fp16(x - hi): 22 to 23 bits of x), two MFMAs onto
+//      one accumulator;
+//   D  the block's sums, multiplied by the block's scale into fp32 sums.
+// At the end a row's sums are multiplied by its power of two. Against 64 bits
+// the results are closer than those of the one-row kernels (2-norm of the
+// error over the result, K = 3136 and 5120: 1.1e-7 and 1.2e-7 against 2.2e-7
+// and 2.5e-7): the products are exact, and the zero points come off the
+// weights exactly instead of as a difference of two large sums.
+//
+// Two launches per call: q4_rows_kernel converts the activation rows into
+// the A operands' lane order in the context's workspace, q4_product_kernel
+// multiplies. A workgroup of the latter stages the weights of 16 or 32
+// columns, all of K, in LDS with copies of whole runs of a column (reading 4
+// blocks at a time straight into the MFMA's lane order touched 3 cache lines
+// for 84 useful bytes of a column and took twice as long), its 8 wavefronts
+// split K and read the A operands of their part from L2.
+#include "nwd_argmax.h"
+#include "nwd_common.h"
+#include "nwd_internal.h"
+
+namespace nwd {
+
+namespace {
+
+// Cells (columns) of up to three projections side by side, the argument block
+// of both kernels.
+struct RowsArgs {
+  Q4Mat m[3];
+  int n_mats;
+  int cols;               // all columns
+  int n_blocks;
+  int rows;               // activation rows of this launch
+  const u32x4* a;         // A operands (q4_rows_kernel)
+  const float* factor;    // [rows] power of two of each row
+  // where the results go
+  int epilogue;           // Q4Epilogue (plain projections)
+  float* y;               // [rows][cols]
+  void* q_out;            // q/k/v: queries and caches
+  f16* k_cache;
+  f16* v_cache;
+  const int32_t* pos;
+  int n_kv, head_dim, cap, q16;
+  int64_t cache_size;     // elements of one cache
+  int* status;
+  unsigned long long* records;  // greedy pick
+  int per_row;
+  int red_offset;  // of the workgroup's sums in LDS
+};
+
+enum RowsKind { kRowsPlain = 0, kRowsQkv = 1, kRowsArgmax = 2 };
+
+// Added to a byte offset, takes a read past its descriptor's range: it
+// returns zeros without a memory access.
+constexpr int kNoRead = 0x7FFFFFFF;
+
+// The matrix that columns col0 .. col0 + 15 lie in (a 16-column tile never
+// straddles two of them: their widths are multiples of 16), col0 made
+// relative to it.
+__device__ inline Q4Mat matrix_of(const RowsArgs& p, int& col0) {
+  Q4Mat m = p.m[0];
+  if (p.n_mats > 1 && col0 >= p.m[0].n) {
+    col0 -= p.m[0].n;
+    m = p.m[1];
+    if (col0 >= p.m[1].n) {
+      col0 -= p.m[1].n;
+      m = p.m[2];
+    }
+  }
+  return m;
+}
+
+__device__ inline f16x2 twice(uint32_t h) {
+  const f16 v = __builtin_bit_cast(f16, (uint16_t)h);
+  return f16x2{v, v};
+}
+__device__ inline f16x2 and_or(uint32_t v, uint32_t mask, uint32_t bits) {
+  uint32_t r;  // one instruction: hipcc makes two of an AND and an OR with literals
+  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "s"(mask), "v"(bits));
+  return __builtin_bit_cast(f16x2, r);
+}
+
+// Eight nibbles less their zero point z as fp16, exactly, in the order
+// 0, 4, 1, 5, 2, 6, 3, 7: a nibble in the low mantissa bits of 1024, or in
+// the next four of 64, is 1024 + n or 64 + n. (The nibbles alone are fp16
+// subnormals, n 2^-24 and n 2^-20, but the MFMAs align such products by
+// their nominal exponent: 4.5e-6 of error against 1.1e-7.)
+__device__ inline f16x8 unpack(uint32_t t, uint32_t z) {
+  constexpr uint32_t k1024 = 0x64006400u, k64 = 0x54005400u;
+  const f16x2 z1024 = twice(z | 0x6400u), z64 = twice(z << 4 | 0x5400u);
+  const uint32_t u = t >> 8;
+  const f16x2 p04 = and_or(t, 0x000F000Fu, k1024) - z1024;
+  const f16x2 p15 = and_or(t, 0x00F000F0u, k64) - z64;
+  const f16x2 p26 = and_or(u, 0x000F000Fu, k1024) - z1024;
+  const f16x2 p37 = and_or(u, 0x00F000F0u, k64) - z64;
+  return f16x8{p04[0], p04[1], p15[0], p15[1], p26[0], p26[1], p37[0], p37[1]};
+}
+
+// ----------------------------------------------------------------- results
+
+// One value of a plain or q/k/v projection to its place (row < p.rows, col
+// < p.cols).
+template <int kKind>
+__device__ inline void put(const RowsArgs& p, int row, int col, float v) {
+  if constexpr (kKind == kRowsPlain) {
+    float* y = p.y + (int64_t)row * p.cols + col;
+    if (p.epilogue == kQ4Relu2) {
+      const float t = fmaxf(v, 0.f);
+      v = t * t;
+    } else if (p.epilogue == kQ4Accumulate) {
+      v = *y + v;  // H[i] = H[i] + B[i]
+    }
+    *y = v;
+  } else if constexpr (kKind == kRowsQkv) {
+    if (col < p.m[0].n) {
+      const int64_t at = (int64_t)row * p.m[0].n + col;
+      if (p.q16)
+        static_cast<f16*>(p.q_out)[at] = (f16)v;
+      else
+        static_cast<float*>(p.q_out)[at] = v;
+      return;
+    }
+    // kv_append (kernels/kv_append.wgsl:12-18), rounded to fp16, at pos[row];
+    // a position outside the cache writes nothing and is reported.
+    col -= p.m[0].n;
+    const bool is_k = col < p.m[1].n;
+    if (!is_k) col -= p.m[1].n;
+    const int t = p.pos[row];
+    if (t < 0 || t >= p.cap) {
+      if (col == 0) atomicOr(p.status, kStatusBadPos);
+      return;
+    }
+    const int64_t at = cache_index_d(row, t, col / p.head_dim, col % p.head_dim, p.n_kv, p.cap, p.head_dim);
+    if (!in_bounds(at, 1, p.cache_size, p.status)) return;
+    (is_k ? p.k_cache : p.v_cache)[at] = (f16)v;
+  }
+}
+
+// ------------------------------------------------------------ activation rows
+
+// One workgroup per activation row: its power of two, and its high and low
+// parts in the lane order of the MFMA A operand. Tile layout (1 KB = 64 lanes
+// of 8 halves): [tile of 16 rows][block][hi, lo], lane (row, g) holding
+// elements 8g .. 8g + 7 of the block in unpack()'s order; packed (up to 8
+// rows), [block] with the high parts as rows 0-7 and the low parts as rows
+// 8-15, one MFMA for both.
+// A row that holds an infinity or a NaN gets the factor NaN: the one-row
+// kernels' sums (nib x - zp x per block) give NaN for such a row too.
+constexpr int kRowsThreads = 256;
+constexpr int kRowsRuns = kQ4MaxBlocks * 4 / kRowsThreads;  // 8-element runs per thread
+
+__global__ __launch_bounds__(kRowsThreads) void q4_rows_kernel(const float* __restrict__ x,
+                                                               int n_blocks, int packed,
+                                                               u32x4* __restrict__ a,
+                                                               float* __restrict__ factor) {
+  __shared__ uint32_t wave_max[kRowsThreads / 64];
+  const int row = blockIdx.x, t = threadIdx.x, runs = n_blocks * 4;
+  const f32x4* xr = reinterpret_cast<const f32x4*>(x + (int64_t)row * n_blocks * 32);
+  f32x4 v[kRowsRuns][2];
+  uint32_t m = 0;
+#pragma unroll
+  for (int j = 0; j < kRowsRuns; ++j) {
+    const int i = t + j * kRowsThreads;
+    if (i < runs) {
+      v[j][0] = xr[2 * i];
+      v[j][1] = xr[2 * i + 1];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < kRowsRuns; ++j) {
+    if (t + j * kRowsThreads < runs) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) m = max(m, __float_as_uint(v[j][e >> 2][e & 3]) & 0x7FFFFFFFu);
+    }
+  }
+#pragma unroll
+  for (int s = 32; s >= 1; s >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, s, 64));
+  if ((t & 63) == 0) wave_max[t >> 6] = m;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kRowsThreads / 64; ++w) m = max(m, wave_max[w]);
+  // 2^e brings the largest magnitude's exponent to 14; e stays where 2^e and
+  // 2^-e are normal numbers.
+  const bool finite = m < 0x7F800000u;
+  const int e = min(141 - (int)(m >> 23), 126);
+  const float up = finite ? __uint_as_float((uint32_t)(e + 127) << 23) : 0.f;
+  if (t == 0)
+    factor[row] = finite ? __uint_as_float((uint32_t)(127 - e) << 23) : __uint_as_float(0x7FC00000u);
+#pragma unroll
+  for (int j = 0; j < kRowsRuns; ++j) {
+    const int i = t + j * kRowsThreads;
+    if (i >= runs) break;
+    f16x8 hi, lo;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int src = (k >> 1) + (k & 1) * 4;  // 0, 4, 1, 5, 2, 6, 3, 7
+      const float f = finite ? v[j][src >> 2][src & 3] * up : 0.f;
+      hi[k] = (f16)f;
+      lo[k] = (f16)(f - (float)hi[k]);
+    }
+    const int blk = i >> 2, g = i & 3;
+    if (packed) {
+      u32x4* o = a + (int64_t)blk * 64 + g * 16 + row;
+      o[0] = __builtin_bit_cast(u32x4, hi);
+      o[8] = __builtin_bit_cast(u32x4, lo);
+    } else {
+      const int64_t at = (int64_t)(row >> 4) * n_blocks + blk;
+      u32x4* o = a + at * 128 + g * 16 + (row & 15);
+      o[0] = __builtin_bit_cast(u32x4, hi);
+      o[64] = __builtin_bit_cast(u32x4, lo);
+    }
+  }
+}
+
+// -------------------------------------------------------------- the products
+
+// A workgroup owns kCols tiles of 16 columns, whose weights, all of K, it
+// stages in LDS at once, and walks row groups of kTiles row tiles (0:
+// packed). Its 8 wavefronts split the blocks of K.
+// LDS of a 16-column tile, in cells (column, block): columns at an odd
+// stride, so that the 16 columns' reads of one block fall on distinct banks.
+__host__ __device__ inline int tile_cells(int n_blocks) { return 16 * (n_blocks | 1); }
+constexpr int kCellBytes = 16 + 4;  // nibbles, scale
+constexpr int kRedPad = 4;
+constexpr int red_floats(int waves, int cols) { return waves * 16 * (cols * 16 + kRedPad); }
+
+template <int kTiles, int kCols, int kWaves, int kKind>
+__global__ __launch_bounds__(kWaves * 64, kTiles == 4 ? 2 : 4) void q4_product_kernel(const RowsArgs p) {
+  constexpr int kThreads = kWaves * 64;
+  constexpr int kPolicy = kKind == kRowsArgmax ? kStreamPolicy : 0;
+  constexpr int kMt = kTiles ? kTiles : 1;                           // row tiles
+  constexpr int kParts = kTiles ? 2 : 1;                             // A operands per tile and block
+  constexpr int kHeld = 8 / (kMt * kParts) < 2 ? 2 : 8 / (kMt * kParts);  // blocks of A operands in flight
+  constexpr int kWgCols = kCols * 16;
+  constexpr int kRows = kTiles ? 16 : 8;  // rows of a tile
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, nb = p.n_blocks;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int stride = nb | 1, cells = tile_cells(nb), col_base = blockIdx.x * kWgCols;
+  u32x4* lds_q = reinterpret_cast<u32x4*>(smem);
+  float* lds_s = reinterpret_cast<float*>(smem + kCols * cells * 16);
+  float* red = reinterpret_cast<float*>(smem + p.red_offset);
+
+  // ---- the weights: nibbles and scales of 64 blocks of a column per copy
+  __amdgpu_buffer_rsrc_t rz[kCols];
+  int zcell[kCols], zlast[kCols];
+#pragma unroll
+  for (int c = 0; c < kCols; ++c) {
+    int col0 = min(col_base + c * 16, p.cols - 1);
+    const Q4Mat m = matrix_of(p, col0);
+    const int n_cells = m.n * nb;  // 16 * n_cells < 2^31 (q4_rows_shape)
+    const auto rq = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(m.quant), 0, n_cells * 16, kBufferWord3);
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(m.scales), 0, n_cells * 4, kBufferWord3);
+    for (int b = 0; b < nb; b += 64) {
+      if (b + lane >= nb) break;
+#pragma unroll
+      for (int i = 0; i < 16 / kWaves; ++i) {
+        const int cc = i * kWaves + wave;
+        if (col0 + cc < m.n) {
+          const int cell = (col0 + cc) * nb + b, at = c * cells + cc * stride + b;
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (lds_void*)(lds_q + at), 16, lane * 16, cell * 16, 0, kPolicy);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(lds_s + at), 4, lane * 4, cell * 4, 0, 0);
+        }
+      }
+    }
+    rz[c] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(m.zp), 0, (n_cells + 1) / 2, kBufferWord3);
+    zcell[c] = min(col0 + (lane & 15), m.n - 1) * nb;
+    zlast[c] = (n_cells + 1) / 2 - 8;
+  }
+
+  // ---- row groups
+  const int first = wave * nb / kWaves, end = (wave + 1) * nb / kWaves;
+  const int groups = (p.rows + kRows * kMt - 1) / (kRows * kMt);
+  const int cell0 = (lane & 15) * stride, g = (lane >> 4) & 3;
+  bool staged = false;
+  for (int group = blockIdx.y; group < groups; group += gridDim.y) {
+    const auto ra = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<u32x4*>(p.a + (int64_t)group * kMt * nb * kParts * 64), 0, kMt * nb * kParts * 1024, kBufferWord3);
+    f16x8 a[kHeld][kMt][kParts];
+    const auto load_a = [&](f16x8 (&dst)[kMt][kParts], int blk) __attribute__((always_inline)) {
+      const int off = blk < end ? 0 : kNoRead;
+#pragma unroll
+      for (int mt = 0; mt < kMt; ++mt)
+#pragma unroll
+        for (int part = 0; part < kParts; ++part)
+          dst[mt][part] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(
+              ra, lane * 16, ((mt * nb + blk) * kParts + part) * 1024 | off, 0));
+    };
+    f32x4 acc[kMt][kCols];
+#pragma unroll
+    for (int mt = 0; mt < kMt; ++mt)
+#pragma unroll
+      for (int c = 0; c < kCols; ++c) acc[mt][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // The lane's column's zero points of 8 blocks from blk on: one 8-byte
+    // read from any nibble offset, moved back where it would pass the end.
+    const auto load_z = [&](u32x2 (&dst)[kCols], int blk) __attribute__((always_inline)) {
+#pragma unroll
+      for (int c = 0; c < kCols; ++c)
+        dst[c] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(
+            rz[c], min((zcell[c] + blk) >> 1, zlast[c]), blk < end ? 0 : kNoRead, 0));
+    };
+    const auto nibbles = [&](const u32x2& v, int c, int blk) __attribute__((always_inline)) {
+      const int byte = (zcell[c] + blk) >> 1;
+      return (uint32_t)(__builtin_bit_cast(uint64_t, v) >>
+                        ((byte - min(byte, zlast[c])) * 8 + ((zcell[c] + blk) & 1) * 4));
+    };
+    // Block blk, the i-th of the zero points in z.
+    const auto block = [&](const f16x8 (&av)[kMt][kParts], int blk, const uint32_t (&z)[kCols], int i) __attribute__((always_inline)) {
+      f16x8 bv[kCols];
+      float s[kCols];
+#pragma unroll
+      for (int c = 0; c < kCols; ++c) {
+        const int cell = c * cells + cell0 + blk;
+        s[c] = lds_s[cell];
+        bv[c] = unpack(reinterpret_cast<const uint32_t*>(lds_q)[cell * 4 + g], (z[c] >> (4 * i)) & 15u);
+      }
+      f32x4 d[kMt][kCols];
+#pragma unroll
+      for (int part = 0; part < kParts; ++part)
+#pragma unroll
+        for (int mt = 0; mt < kMt; ++mt)
+#pragma unroll
+          for (int c = 0; c < kCols; ++c)
+            d[mt][c] = mfma16x16x32(av[mt][part], bv[c], part ? d[mt][c] : f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+      for (int mt = 0; mt < kMt; ++mt)
+#pragma unroll
+        for (int c = 0; c < kCols; ++c)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[mt][c][r] = fmaf(s[c], d[mt][c][r], acc[mt][c][r]);
+    };
+#pragma unroll
+    for (int i = 0; i < kHeld; ++i) load_a(a[i], first + i);
+    u32x2 zv[kCols];
+    load_z(zv, first);
+    if (!staged) {
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the copies into LDS
+      __syncthreads();
+      staged = true;
+    }
+    for (int blk = first; blk < end; blk += 8) {
+      uint32_t z[kCols];
+#pragma unroll
+      for (int c = 0; c < kCols; ++c) z[c] = nibbles(zv[c], c, blk);
+      load_z(zv, blk + 8);
+      if (blk + 8 <= end) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          block(a[i % kHeld], blk + i, z, i);
+          load_a(a[i % kHeld], blk + i + kHeld);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          if (blk + i < end) block(a[i % kHeld], blk + i, z, i);
+          if (kHeld < 8 && blk + i + kHeld < end) load_a(a[i % kHeld], blk + i + kHeld);
+        }
+      }
+    }
+
+    // The wavefronts' sums, added in wavefront order, one row tile at a time.
+#pragma unroll
+    for (int mt = 0; mt < kMt; ++mt) {
+      __syncthreads();
+#pragma unroll
+      for (int c = 0; c < kCols; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          red[(wave * 16 + (lane >> 4) * 4 + r) * (kWgCols + kRedPad) + c * 16 + (lane & 15)] = acc[mt][c][r];
+      __syncthreads();
+#pragma unroll
+      for (int e = 0; e < kRows * kWgCols; e += kThreads) {
+        const int r = (e + tid) / kWgCols, cc = (e + tid) % kWgCols;
+        const int row = (group * kMt + mt) * kRows + r, cl = col_base + cc;
+        const bool live = r < kRows && row < p.rows && cl < p.cols;
+        float v = 0.f;
+        if (r < kRows) {
+#pragma unroll
+          for (int k = 0; k < kWaves; ++k) {
+            v += red[(k * 16 + r) * (kWgCols + kRedPad) + cc];
+            if constexpr (!kTiles) v += red[(k * 16 + r + 8) * (kWgCols + kRedPad) + cc];
+          }
+        }
+        if (live) v *= p.factor[row];
+        if constexpr (kKind == kRowsArgmax) {  // one record per row and workgroup
+          if (live && p.y) p.y[(int64_t)row * p.cols + cl] = v;
+          unsigned long long best = live ? argmax_enc(v, cl, argmax_shape(p.cols)) : 0ull;
+#pragma unroll
+          for (int m = kWgCols / 2; m >= 1; m >>= 1) {
+            const unsigned long long o = __shfl_xor(best, m, 64);
+            best = o > best ? o : best;
+          }
+          if (cc == 0 && r < kRows && row < p.rows) p.records[(int64_t)row * p.per_row + blockIdx.x] = best;
+        } else {
+          if (live) put<kKind>(p, row, cl, v);
+        }
+      }
+    }
+  }
+}
+
+// ------------------------------------------------------------------- launch
+
+constexpr int kPackedRows = 8;
+
+// Row tiles (0: packed), column tiles and wavefronts of a workgroup, and the
+// workgroups that share a column range's row groups.
+struct RowsPlan {
+  int tiles, cols, waves, split;
+};
+
+// Row tiles: as few as hold the rows, up to 4 (64 rows: a wavefront's sums,
+// operands and products then fill its 256 registers). Two column tiles halve
+// what a workgroup reads of the A operands per column, which L2 bounds: for
+// wide projections, which fill the chip many times over, and with 4 row
+// tiles where the workgroups still fill half of it. us per call, one tile
+// against two: K = 3136, 64 rows, 7168 columns 27.1 against 19.8; 131072
+// columns, 4 and 16 rows 88.5 against 76.2 and 115 against 108; but K =
+// 3136, 16 and 32 rows, 7168 columns 12.6 against 12.9 and 15.3 against
+// 16.2, K = 5120, 16 and 64 rows, 3136 columns 11.4 against 14.2 and 22.4
+// against 24.2.
+// Wavefronts: 8, or 4 where two such workgroups of 64 rows then fit a CU (by
+// their LDS) and the launch has them: 512 rows, K = 3136, 5120 columns 66.5
+// against 76.6; one workgroup per CU loses with 4 (K = 5120, 3136 columns
+// 88.5 against 76.1, 1024 columns 27.3 against 25.0).
+// Split: the launch takes rounds of as many workgroups as fit the chip; the
+// split with the fewest rounds times row groups (and half a group for the
+// weights) wins. 512 rows, 8 wavefronts, split 8 / 4 / 2: K = 3136, 5120
+// columns 76.6 / 80.0 / 99.2 us; K = 5120, 3136 columns 90.5 / 82.5 / 76.1;
+// K = 3136, 1024 columns 25.0 / 34.9 / 55.8.
+RowsPlan rows_plan(int cols, int n_blocks, int rows) {
+  constexpr int kCus = 256, kWide = 16384;
+  RowsPlan r;
+  r.tiles = rows <= kPackedRows ? 0 : (rows <= 16 ? 1 : (rows <= 32 ? 2 : 4));
+  const int per = r.tiles ? 16 * r.tiles : kPackedRows, groups = (rows + per - 1) / per;
+  const int64_t pairs = (cols + 31) / 32;
+  r.cols = n_blocks <= 160 && (cols >= kWide || (r.tiles == 4 && pairs * groups >= kCus / 2)) ? 2 : 1;
+  const int64_t wgs = r.cols == 2 ? pairs : (cols + 15) / 16;
+  r.waves = r.tiles == 4 && n_blocks <= 100 && wgs * groups >= 2 * kCus ? 4 : 8;
+  const int64_t slots = r.waves == 4 ? 2 * kCus : kCus;
+  r.split = 1;
+  double best = 0;
+  for (int s = 1; s <= groups && s <= 64; ++s) {
+    const double t = (double)((wgs * s + slots - 1) / slots) * ((groups + s - 1) / s + 0.5);
+    if (s == 1 || t < best) {
+      best = t;
+      r.split = s;
+    }
+  }
+  return r;
+}
+
+// Bytes of A operands and factors that `rows` rows of a launch take.
+size_t factor_offset(int rows, int n_blocks) {
+  return rows <= kPackedRows ? (size_t)n_blocks * 1024 : (size_t)((rows + 63) / 64 * 4) * n_blocks * 2048;
+}
+size_t rows_bytes(int rows, int n_blocks) {
+  return factor_offset(rows, n_blocks) + (size_t)((rows + 3) / 4) * 16;
+}
+
+// Rows per launch within the scratch: all of them, or a multiple of 64 or 8.
+int rows_per_launch(int rows, int n_blocks, size_t scratch) {
+  if (rows_bytes(rows, n_blocks) <= scratch) return rows;
+  int r = rows / 64 * 64;
+  while (r > 64 && rows_bytes(r, n_blocks) > scratch) r -= 64;
+  if (r >= 64 && rows_bytes(r, n_blocks) <= scratch) return r;
+  return rows_bytes(kPackedRows, n_blocks) <= scratch ? kPackedRows : 0;
+}
+
+template <int kKind>
+hipError_t launch_rows(RowsArgs p, const float* x, Q4Scratch scratch, hipStream_t stream) {
+  const int rows = p.rows, nb = p.n_blocks;
+  p.a = reinterpret_cast<const u32x4*>(scratch.base);
+  float* factor = reinterpret_cast<float*>(static_cast<char*>(scratch.base) + factor_offset(rows, nb));
+  p.factor = factor;
+  const RowsPlan plan = rows_plan(p.cols, nb, rows);
+  q4_rows_kernel<<<rows, kRowsThreads, 0, stream>>>(x, nb, plan.tiles == 0 ? 1 : 0,
+                                                    static_cast<u32x4*>(scratch.base), factor);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const int wg_cols = plan.cols * 16, wg_rows = plan.tiles ? 16 * plan.tiles : kPackedRows;
+  const int groups = (rows + wg_rows - 1) / wg_rows, split = groups < plan.split ? groups : plan.split;
+  const dim3 grid((p.cols + wg_cols - 1) / wg_cols, split);
+  p.per_row = grid.x;
+  // The sums may overwrite the weights where no other row group follows.
+  const int weights = plan.cols * tile_cells(nb) * kCellBytes, sums = red_floats(plan.waves, plan.cols) * 4;
+  p.red_offset = split == groups ? 0 : weights;
+  const int lds = split == groups ? (weights > sums ? weights : sums) : weights + sums;
+#define NWD_ROWS_CASE(T, C, W)                                                                \
+  if (plan.tiles == T && plan.cols == C && plan.waves == W) {                                 \
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(q4_product_kernel<T, C, W, kKind>), \
+                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);          \
+    if (e != hipSuccess) return e;                                                            \
+    q4_product_kernel<T, C, W, kKind><<<grid, W * 64, lds, stream>>>(p);                      \
+    return hipGetLastError();                                                                 \
+  }
+  NWD_ROWS_CASE(0, 1, 8) NWD_ROWS_CASE(0, 2, 8) NWD_ROWS_CASE(1, 1, 8) NWD_ROWS_CASE(1, 2, 8)
+  NWD_ROWS_CASE(2, 1, 8) NWD_ROWS_CASE(2, 2, 8) NWD_ROWS_CASE(4, 1, 8) NWD_ROWS_CASE(4, 2, 8)
+  NWD_ROWS_CASE(4, 1, 4) NWD_ROWS_CASE(4, 2, 4)
+#undef NWD_ROWS_CASE
+  return hipErrorInvalidValue;
+}
+
+RowsArgs rows_args(const Q4Mat* m, int n_mats, int n_blocks) {
+  RowsArgs p{};
+  p.n_mats = n_mats;
+  for (int i = 0; i < n_mats; ++i) {
+    p.m[i] = m[i];
+    p.cols += m[i].n;
+  }
+  p.n_blocks = n_blocks;
+  return p;
+}
+
+}  // namespace
+
+bool q4_rows_shape(int n, int narrowest, int n_blocks, int rows, bool pick, Q4Scratch scratch) {
+  const int64_t cells = (int64_t)n * n_blocks;
+  return rows >= 2 && cells * rows >= (pick && n >= 16384 ? 6000000 : 1500000) &&
+         (int64_t)narrowest * n_blocks >= 16 && cells * 16 < ((int64_t)1 << 31) - (1 << 20) &&
+         rows_per_launch(rows, n_blocks, scratch.bytes) > 0;
+}
+
+hipError_t launch_q4_rows_gemv(const float* x, const Q4Mat& w, int n_blocks, float* y, int rows,
+                               int epilogue, Q4Scratch scratch, hipStream_t stream) {
+  const int per = rows_per_launch(rows, n_blocks, scratch.bytes);
+  for (int r = 0; r < rows; r += per) {
+    RowsArgs p = rows_args(&w, 1, n_blocks);
+    p.rows = rows - r < per ? rows - r : per;
+    p.epilogue = epilogue;
+    p.y = y + (int64_t)r * w.n;
+    const hipError_t e = launch_rows<kRowsPlain>(p, x + (int64_t)r * n_blocks * 32, scratch, stream);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+hipError_t launch_q4_rows_qkv(const Shape& s, const float* x, const Q4Mat& wq, const Q4Mat& wk,
+                              const Q4Mat& wv, int n_blocks, void* q_out, void* k_cache,
+                              void* v_cache, const int32_t* pos, int batch, int* status,
+                              Q4Scratch scratch, hipStream_t stream) {
+  const Q4Mat m[3] = {wq, wk, wv};
+  const int per = rows_per_launch(batch, n_blocks, scratch.bytes);
+  const int64_t seq = (int64_t)s.n_kv * s.cap * s.head_dim;  // cache elements per sequence
+  for (int r = 0; r < batch; r += per) {
+    RowsArgs p = rows_args(m, 3, n_blocks);
+    p.rows = batch - r < per ? batch - r : per;
+    p.q_out = static_cast<char*>(q_out) + (int64_t)r * wq.n * (s.q16 ? 2 : 4);
+    p.k_cache = static_cast<f16*>(k_cache) + r * seq;
+    p.v_cache = static_cast<f16*>(v_cache) + r * seq;
+    p.pos = pos + r;
+    p.n_kv = s.n_kv;
+    p.head_dim = s.head_dim;
+    p.cap = s.cap;
+    p.q16 = s.q16;
+    p.cache_size = p.rows * seq;
+    p.status = status;
+    const hipError_t e = launch_rows<kRowsQkv>(p, x + (int64_t)r * n_blocks * 32, scratch, stream);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+hipError_t launch_q4_rows_argmax(const float* x, const Q4Mat& w, int n_blocks, float* logits,
+                                 uint32_t* out, int batch, unsigned long long* records,
+                                 Q4Scratch scratch, hipStream_t stream) {
+  const int per = rows_per_launch(batch, n_blocks, scratch.bytes);
+  for (int r = 0; r < batch; r += per) {
+    RowsArgs p = rows_args(&w, 1, n_blocks);
+    p.rows = batch - r < per ? batch - r : per;
+    p.y = logits ? logits + (int64_t)r * w.n : nullptr;
+    p.records = records;
+    hipError_t e = launch_rows<kRowsArgmax>(p, x + (int64_t)r * n_blocks * 32, scratch, stream);
+    const int wg_cols = 16 * rows_plan(w.n, n_blocks, p.rows).cols;  // one record each
+    const int per_row = (w.n + wg_cols - 1) / wg_cols;
+    if (e == hipSuccess) e = launch_argmax_merge(records, per_row, w.n, out + r, p.rows, stream);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+}  // namespace nwd

@@ -1,0 +1,190 @@
+"""Parity of the 4-bit projections of several activation rows (the matrix-core
+kernels of nwd_q4_rows.hip) with float64, through the C ABI.
+
+Bars: |y - y64| <= 1e-6 sum_k |w_k a_k| (the one-row kernels' bar; their
+activations enter as fp16 high and low parts, within 2^-22 of each, and 32
+products are summed at a time); a row that holds an infinity or a NaN is NaN,
+as on the one-row kernels; cache rows within one fp16 ulp; the picked token
+is the largest logit.
+
+Sizes: the smallest and largest row counts of each row tiling (packed up to
+8, then 16, 32 and 64 rows, several groups of 64), column counts that leave a
+remainder of the 16- and 32-column tiles, odd block counts, one block, and
+the largest K. Each product of rows and cells is past the 1.5 million from
+which these kernels run.
+"""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+import nwd_attn as nw  # noqa: E402
+from gpu_util import dev, host, pos_tensor, say  # noqa: E402
+from q4_cases import dequant_f64, random_q4, rng  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+TOL_REL = 1e-6
+D = 128
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    if not torch.cuda.is_available():
+        pytest.fail("GPU tests need a visible MI355X")
+    nw.load_library()
+
+
+class Q4:
+    def __init__(self, g, n, n_blocks):
+        quant, scales, zp = random_q4(g, n, n_blocks)
+        self.t = (dev(quant), dev(scales), dev(zp))
+        self.w = nw.q4_weight(*self.t, n, n_blocks)
+        self.dense = torch.from_numpy(dequant_f64(quant, scales, zp)).cuda()
+
+    def f64(self, x):
+        x = torch.from_numpy(np.asarray(x, np.float64)).cuda()
+        return host(x @ self.dense.t()), host(x.abs() @ self.dense.abs().t())
+
+
+def _ctx(H=32, Hkv=8, cap=512, B=64, q="f32", Dh=D):
+    return nw.AttnContext(H, Hkv, cap, head_dim=Dh, max_batch=B, q_dtype=q, o_dtype="f32",
+                          kv_dtype="f32")
+
+
+@pytest.mark.parametrize("n,n_blocks,rows", [
+    (8192, 98, 2),     # packed: the smallest
+    (1953, 98, 8),     # packed, full; one column past a tile
+    (2050, 97, 9),     # one tile of 16, odd block count
+    (1000, 98, 16),
+    (1007, 98, 17),    # two tiles
+    (520, 98, 32),
+    (3136, 160, 33),   # four tiles, mostly padding; K = 5120
+    (7168, 98, 64),    # two column tiles per workgroup
+    (300, 98, 65),     # a second group of one row
+    (5120, 98, 300),   # four wavefronts per workgroup
+    (3136, 160, 200),  # a workgroup walks several groups
+    (37, 130, 320),    # few columns
+    (64, 256, 130),    # the largest K
+    (48, 1, 40000),    # one block: most wavefronts have none
+    (777, 5, 500),
+])
+def test_rows_match_float64(n, n_blocks, rows):
+    say(f"q4 rows n={n} n_blocks={n_blocks} rows={rows}")
+    g = rng(900 + n + rows)
+    w = Q4(g, n, n_blocks)
+    x = g.standard_normal((rows, 32 * n_blocks)).astype(np.float32)
+    prev = g.standard_normal((rows, n)).astype(np.float32)
+    y = torch.full((rows, n), float("nan"), dtype=torch.float32, device="cuda")
+    relu, acc = torch.empty_like(y), dev(prev)
+    with _ctx() as ctx:
+        ctx.q4_gemv(dev(x), w.w, y, rows)
+        ctx.q4_gemv(dev(x), w.w, relu, rows, nw.NWD_Q4_RELU2)
+        ctx.q4_gemv(dev(x), w.w, acc, rows, nw.NWD_Q4_ACCUMULATE)
+        got = host(y)
+    y64, bound = w.f64(x)
+    assert np.all(np.abs(got - y64) <= TOL_REL * bound)
+    t = np.maximum(got, np.float32(0))
+    np.testing.assert_array_equal(host(relu), t * t)
+    np.testing.assert_array_equal(host(acc), prev + got)
+
+
+def test_rows_in_small_workspace():
+    """A context whose workspace holds few activation rows: the call goes
+    through it in several launches."""
+    n, n_blocks, rows = 1024, 256, 150
+    say(f"q4 rows in a small workspace, rows={rows}")
+    g = rng(950)
+    w = Q4(g, n, n_blocks)
+    x = g.standard_normal((rows, 32 * n_blocks)).astype(np.float32)
+    for heads in (1, 2, 4):
+        y = torch.full((rows, n), float("nan"), dtype=torch.float32, device="cuda")
+        with _ctx(heads, heads, 16, 1) as ctx:
+            ctx.q4_gemv(dev(x), w.w, y, rows)
+            got = host(y)
+        y64, bound = w.f64(x)
+        assert np.all(np.abs(got - y64) <= TOL_REL * bound), heads
+
+
+def test_rows_ranges_and_non_finite():
+    """Rows at the ends of float32's range, of zeros, and with an infinity or
+    a NaN, beside ordinary ones."""
+    say("q4 rows: ranges, infinities, NaN")
+    n, n_blocks, rows = 1200, 98, 14
+    g = rng(951)
+    w = Q4(g, n, n_blocks)
+    x = g.standard_normal((rows, 32 * n_blocks)).astype(np.float32)
+    x[1] *= np.float32(1e30)
+    x[2] *= np.float32(1e-30)
+    x[3] = 0
+    x[4, 7] = np.inf
+    x[5, 3000] = np.nan
+    x[6, 100] = -np.inf
+    x[7] *= np.float32(1e-41) / np.float32(1e-3)  # subnormals
+    x[8, 5] = 3e4  # one large element among small ones
+    y = torch.zeros((rows, n), dtype=torch.float32, device="cuda")
+    with _ctx() as ctx:
+        ctx.q4_gemv(dev(x), w.w, y, rows)
+        got = host(y)
+    bad = [4, 5, 6]
+    assert np.all(np.isnan(got[bad]))
+    fine = [b for b in range(rows) if b not in bad]
+    y64, bound = w.f64(x[fine])
+    # a subnormal result is within half its last place, 2^-150
+    assert np.all(np.abs(got[fine] - y64) <= TOL_REL * bound + 2.0 ** -149)
+
+
+@pytest.mark.parametrize("H,Hkv,q,Dh,B", [(40, 8, "f32", 128, 3), (32, 8, "f16", 128, 12),
+                                          (14, 2, "f32", 64, 40), (6, 2, "f16", 96, 64)])
+def test_qkv_rows(H, Hkv, q, Dh, B):
+    """q, k and v through the fused projection; the last sequence's position
+    is outside its cache: nothing is written there and it is reported."""
+    say(f"qkv rows H={H} Hkv={Hkv} D={Dh} B={B}")
+    g = rng(960 + B)
+    cap, nb = 24, 98
+    wq, wk, wv = Q4(g, H * Dh, nb), Q4(g, Hkv * Dh, nb), Q4(g, Hkv * Dh, nb)
+    x = g.standard_normal((B, 32 * nb)).astype(np.float32)
+    pos = [int(v) for v in g.integers(0, cap, size=B)]
+    pos[-1] = cap
+    canary = -7.5
+    with _ctx(H, Hkv, cap, B, q, Dh) as ctx:
+        kc = torch.full((B, Hkv, cap, Dh), canary, dtype=torch.float16, device="cuda")
+        vc = kc.clone()
+        qo = torch.empty((B, H, Dh), dtype=torch.float32 if q == "f32" else torch.float16, device="cuda")
+        ctx.qkv_append(dev(x), wq.w, wk.w, wv.w, qo, kc, vc, pos_tensor(pos), B)
+        assert ctx.device_status() == nw.NWD_ERR_DEVICE
+        assert ctx.device_status() == nw.NWD_OK
+        qh, kh, vh = host(qo).astype(np.float64), host(kc), host(vc)
+
+    def ulp(v):
+        h = v.astype(np.float16)
+        return np.abs((np.nextafter(h, np.float16(np.inf)) - h).astype(np.float64))
+
+    y64, bound = wq.f64(x)
+    assert np.all(np.abs(qh.reshape(B, -1) - y64) <= TOL_REL * bound + (ulp(y64) if q == "f16" else 0))
+    for w, c in ((wk, kh), (wv, vh)):
+        y64, bound = w.f64(x)
+        for b in range(B):
+            row = slice(0, 0) if pos[b] == cap else slice(pos[b], pos[b] + 1)
+            got = c[b, :, row, :].astype(np.float64).reshape(-1)
+            if got.size:
+                assert np.all(np.abs(got - y64[b]) <= TOL_REL * bound[b] + ulp(y64[b])), b
+            assert np.all(np.delete(c[b], row, axis=1) == np.float16(canary)), b
+
+
+@pytest.mark.parametrize("n,n_blocks,rows", [(20011, 98, 4), (20011, 98, 16), (16384, 97, 20), (33000, 33, 70)])
+def test_lm_head_rows(n, n_blocks, rows):
+    say(f"lm_head rows n={n} n_blocks={n_blocks} rows={rows}")
+    g = rng(970 + rows)
+    w = Q4(g, n, n_blocks)
+    x = g.standard_normal((rows, 32 * n_blocks)).astype(np.float32)
+    logits = torch.empty((rows, n), dtype=torch.float32, device="cuda")
+    token = torch.full((2, rows), -1, dtype=torch.int32, device="cuda")
+    with _ctx() as ctx:
+        ctx.lm_head_argmax(dev(x), w.w, token[0], logits, rows)
+        ctx.lm_head_argmax(dev(x), w.w, token[1], None, rows)
+        got, tok = host(logits), host(token)
+    y64, bound = w.f64(x)
+    assert np.all(np.abs(got - y64) <= TOL_REL * bound)
+    np.testing.assert_array_equal(tok[0], np.argmax(got, axis=1))
+    np.testing.assert_array_equal(tok[1], tok[0])
