@@ -185,12 +185,6 @@ __device__ inline f32x4 mfma16x16x32(f16x8 a, f16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
 
-// D = A B + C on v_mfma_f32_16x16x4_f32, in fp32: lane (r, q) holds A[r][q],
-// B[q][r] and D[4q .. 4q+3][r].
-__device__ inline f32x4 mfma16x16x4(float a, float b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
 __device__ inline float dot2(f16x2 a, f16x2 b, float c) {
   return __builtin_amdgcn_fdot2(a, b, c, false);
 }

@@ -79,9 +79,9 @@ __device__ inline Q4Mat matrix_of(const RowsArgs& p, int& col0) {
   return m;
 }
 
-__device__ inline f16x2 twice(uint32_t h) {
-  const f16 v = __builtin_bit_cast(f16, (uint16_t)h);
-  return f16x2{v, v};
+__device__ inline f16x2 twice(uint32_t h) {  // the low half in both
+  const f16x2 v = __builtin_bit_cast(f16x2, h);
+  return __builtin_shufflevector(v, v, 0, 0);
 }
 __device__ inline f16x2 and_or(uint32_t v, uint32_t mask, uint32_t bits) {
   uint32_t r;  // one instruction: hipcc makes two of an AND and an OR with literals
@@ -408,6 +408,202 @@ __global__ __launch_bounds__(kWaves * 64, kTiles == 4 ? 2 : 4) void q4_product_k
   }
 }
 
+// ------------------------------------------------------- wide greedy picks
+
+// lm_head with the pick, up to 48 rows: one persistent workgroup per CU. Its
+// 8 wavefronts split K and hold their part of one row tile's A operands in
+// registers for the whole launch (read per 32 columns, as above, they were
+// more L2 traffic than the weights); the weights of the next 32 columns, one
+// run of memory, lie in the other LDS buffer and those after it are on their
+// way in registers. Row tiles share the workgroups out, side
+// by side over the same columns, so that L2 and the Infinity Cache serve the
+// weights' second reading. A thread keeps the best of its logits of a row;
+// one record per row and workgroup. 131072 x 3136, us per call against the
+// kernel above: 4 rows 88 to 72, 16 rows 120 to 81, 32 rows 218 to 142. Its
+// products alone take 44 of them, its reads 55 (4.8 TB/s).
+constexpr int kPickWaves = 8;
+constexpr int kPickThreads = kPickWaves * 64;
+constexpr int kPickCols = 32;
+constexpr int kPickBlocks = 13;                  // of K per wavefront, at most
+constexpr int kPickMaxBlocks = 8 * kPickBlocks;  // 104: K <= 3328
+constexpr int kPickLoads = kPickCols * kPickMaxBlocks / kPickThreads + 1;
+static_assert((kPickBlocks + 3) / 4 * 2 >= kPickLoads, "two requests beside every four blocks");
+constexpr int kPickRed = kPickWaves * 16 * (kPickCols + kRedPad);  // floats
+constexpr int pick_lds(int n_blocks) { return 2 * kPickCols * (n_blocks | 1) * kCellBytes + kPickRed * 4; }
+
+template <int kTiles>
+__global__ __launch_bounds__(kPickThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void q4_pick_kernel(
+    const RowsArgs p, int row_tiles) {
+  constexpr int kParts = kTiles ? 2 : 1;
+  constexpr int kRows = kTiles ? 16 : 8;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, nb = p.n_blocks;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tile = blockIdx.x % row_tiles, slot = blockIdx.x / row_tiles;
+  const int slots = gridDim.x / row_tiles;  // workgroups of a row tile
+  const int groups = (p.cols + kPickCols - 1) / kPickCols;
+  const int stride = nb | 1, buffer = kPickCols * stride * kCellBytes;
+  float* red = reinterpret_cast<float*>(smem + 2 * buffer);
+  const Q4Mat m = p.m[0];
+  const int n_cells = m.n * nb;  // 16 * n_cells < 2^31 (q4_rows_shape)
+  const auto rq = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(m.quant), 0, n_cells * 16, kBufferWord3);
+  const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(m.scales), 0, n_cells * 4, kBufferWord3);
+  const auto rz = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(m.zp), 0, (n_cells + 1) / 2, kBufferWord3);
+  const int zlast = (n_cells + 1) / 2 - 8;
+  const int first = wave * nb / kPickWaves, end = (wave + 1) * nb / kPickWaves;
+
+  // Cell tid + 512 i of a group's run of 32 nb cells, and where it goes.
+  int to[kPickLoads];
+  const int cells = kPickCols * nb;
+#pragma unroll
+  for (int i = 0; i < kPickLoads; ++i) {
+    const int idx = tid + i * kPickThreads, c = idx / nb;
+    to[i] = idx < cells ? c * stride + idx - c * nb : -1;
+  }
+  u32x4 wq[kPickLoads];
+  float ws[kPickLoads];
+  u32x2 zn[2][2];     // [column tile][blocks first .. + 7, first + 8 .. + 15]
+  uint32_t zv[2][2], znext[2][2];  // zero points of those blocks, a nibble each
+  // Requests i and i + 1 of a group's, the zero points with the last. A
+  // group's requests do not fit the memory path's queues at once: issued
+  // together they held the wavefronts up for as long as the products take.
+  const auto load_w = [&](int group, int first_i) __attribute__((always_inline)) {
+    const int base = group * cells;  // past the last column: out of range, zeros
+    const int off = group < groups ? 0 : kNoRead;
+#pragma unroll
+    for (int i = first_i; i < first_i + 2; ++i) {
+      if (i >= kPickLoads) break;
+      const int cell = base + tid + i * kPickThreads;
+      const bool in = to[i] >= 0 && cell < n_cells;
+      wq[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+          rq, in ? cell * 16 : kNoRead, off, kStreamPolicy));
+      ws[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, in ? cell * 4 : kNoRead, off, 0));
+    }
+    if (first_i + 2 < kPickLoads) return;
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int cell = min(group * kPickCols + c * 16 + (lane & 15), m.n - 1) * nb + first + 8 * h;
+        zn[c][h] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(
+            rz, min(cell >> 1, zlast), first + 8 * h < end ? off : kNoRead, 0));
+      }
+  };
+  const auto load_all = [&](int group) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kPickLoads; i += 2) load_w(group, i);
+  };
+  const auto store_w = [&](int buf, int group) __attribute__((always_inline)) {
+    u32x4* q = reinterpret_cast<u32x4*>(smem + buf * buffer);
+    float* s = reinterpret_cast<float*>(smem + buf * buffer + kPickCols * stride * 16);
+#pragma unroll
+    for (int i = 0; i < kPickLoads; ++i)
+      if (to[i] >= 0) {
+        q[to[i]] = wq[i];
+        s[to[i]] = ws[i];
+      }
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int cell = min(group * kPickCols + c * 16 + (lane & 15), m.n - 1) * nb + first + 8 * h, byte = cell >> 1;
+        znext[c][h] = (uint32_t)(__builtin_bit_cast(uint64_t, zn[c][h]) >>
+                                 ((byte - min(byte, zlast)) * 8 + (cell & 1) * 4));
+      }
+  };
+
+  f16x8 a[kPickBlocks][kParts];
+  const auto ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<u32x4*>(p.a + (int64_t)tile * nb * kParts * 64), 0,
+                                                    nb * kParts * 1024, kBufferWord3);
+  load_all(slot);
+#pragma unroll
+  for (int b = 0; b < kPickBlocks; ++b)
+#pragma unroll
+    for (int part = 0; part < kParts; ++part)
+      a[b][part] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(
+          ra, lane * 16, first + b < end ? ((first + b) * kParts + part) * 1024 : kNoRead, 0));
+  // The thread's logit of a group: row tid / 32 of the tile, column tid % 32.
+  const int r = tid / kPickCols, cc = tid % kPickCols, row = tile * kRows + r;
+  const bool live_row = r < kRows && row < p.rows;
+  const float factor = live_row ? p.factor[row] : 0.f;
+  const ArgmaxShape shape = argmax_shape(p.cols);
+  unsigned long long best = 0ull;
+  const auto step_z = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) zv[c][h] = znext[c][h];
+  };
+  store_w(0, slot);
+  step_z();
+  load_all(slot + slots);
+  __syncthreads();
+
+  int buf = 0;
+  for (int group = slot; group < groups; group += slots, buf ^= 1) {
+    store_w(buf ^ 1, group + slots);  // requested an iteration ago
+    const uint32_t* q = reinterpret_cast<const uint32_t*>(smem + buf * buffer);
+    const float* s = reinterpret_cast<const float*>(smem + buf * buffer + kPickCols * stride * 16);
+    f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+    const auto block = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int cell = (c * 16 + (lane & 15)) * stride + first + b;
+        const f16x8 bv = unpack(q[cell * 4 + (lane >> 4)], (zv[c][b / 8] >> (4 * (b % 8))) & 15u);
+        f32x4 d = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int part = 0; part < kParts; ++part) d = mfma16x16x32(a[b][part], bv, d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[c][e] = fmaf(s[cell], d[e], acc[c][e]);
+      }
+    };
+    // four blocks to a branch, so that their reads and products overlap
+#pragma unroll
+    for (int b = 0; b < kPickBlocks; b += 4) {
+      load_w(group + 2 * slots, b / 2);
+      __builtin_amdgcn_sched_barrier(0);
+      if (b + 4 <= kPickBlocks && first + b + 4 <= end) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (b + i < kPickBlocks) block(b + i);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (b + i < kPickBlocks && first + b + i < end) block(b + i);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        red[(wave * 16 + (lane >> 4) * 4 + e) * (kPickCols + kRedPad) + c * 16 + (lane & 15)] = acc[c][e];
+    step_z();
+    __syncthreads();
+    const int cl = group * kPickCols + cc;
+    if (r < kRows) {
+      float v = 0.f;
+#pragma unroll
+      for (int k = 0; k < kPickWaves; ++k) {
+        v += red[(k * 16 + r) * (kPickCols + kRedPad) + cc];
+        if constexpr (!kTiles) v += red[(k * 16 + r + 8) * (kPickCols + kRedPad) + cc];
+      }
+      v *= factor;
+      if (live_row && cl < p.cols) {
+        if (p.y) p.y[(int64_t)row * p.cols + cl] = v;
+        const unsigned long long e = argmax_enc(v, cl, shape);
+        best = e > best ? e : best;
+      }
+    }
+    __syncthreads();  // the sums are read
+  }
+#pragma unroll
+  for (int i = kPickCols / 2; i >= 1; i >>= 1) {
+    const unsigned long long o = __shfl_xor(best, i, 64);
+    best = o > best ? o : best;
+  }
+  if (cc == 0 && live_row) p.records[(int64_t)row * p.per_row + slot] = best;
+}
+
 // ------------------------------------------------------------------- launch
 
 constexpr int kPackedRows = 8;
@@ -459,6 +655,19 @@ RowsPlan rows_plan(int cols, int n_blocks, int rows) {
   return r;
 }
 
+// The wide pick: its grid, which picks it takes, and its records per row
+// (one per workgroup of a row tile). The limit of K is its registers'; of
+// rows, 131072 x 3136: 48 rows 203 against 210 us, 64 rows 258 against 222.
+constexpr int kPickGrid = 256;
+bool pick_wide(int cols, int n_blocks, int rows) {
+  return cols >= 16384 && n_blocks <= kPickMaxBlocks && rows <= 48;
+}
+int pick_records(int rows) {
+  const int tiles = rows <= kPackedRows ? 1 : (rows + 15) / 16;
+  return kPickGrid / tiles;
+}
+static_assert(pick_lds(kPickMaxBlocks) <= 160 * 1024, "the weights of two groups and the sums fit a CU");
+
 // Bytes of A operands and factors that `rows` rows of a launch take.
 size_t factor_offset(int rows, int n_blocks) {
   return rows <= kPackedRows ? (size_t)n_blocks * 1024 : (size_t)((rows + 63) / 64 * 4) * n_blocks * 2048;
@@ -482,6 +691,26 @@ hipError_t launch_rows(RowsArgs p, const float* x, Q4Scratch scratch, hipStream_
   p.a = reinterpret_cast<const u32x4*>(scratch.base);
   float* factor = reinterpret_cast<float*>(static_cast<char*>(scratch.base) + factor_offset(rows, nb));
   p.factor = factor;
+  if constexpr (kKind == kRowsArgmax) {
+    if (pick_wide(p.cols, nb, rows)) {
+      const bool packed = rows <= kPackedRows;
+      const int tiles = packed ? 1 : (rows + 15) / 16;
+      q4_rows_kernel<<<rows, kRowsThreads, 0, stream>>>(x, nb, packed ? 1 : 0,
+                                                        static_cast<u32x4*>(scratch.base), factor);
+      hipError_t e = hipGetLastError();
+      const void* kern = packed ? reinterpret_cast<const void*>(q4_pick_kernel<0>)
+                                : reinterpret_cast<const void*>(q4_pick_kernel<1>);
+      if (e == hipSuccess)
+        e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+      if (e != hipSuccess) return e;
+      p.per_row = pick_records(rows);
+      if (packed)
+        q4_pick_kernel<0><<<tiles * p.per_row, kPickThreads, pick_lds(nb), stream>>>(p, tiles);
+      else
+        q4_pick_kernel<1><<<tiles * p.per_row, kPickThreads, pick_lds(nb), stream>>>(p, tiles);
+      return hipGetLastError();
+    }
+  }
   const RowsPlan plan = rows_plan(p.cols, nb, rows);
   q4_rows_kernel<<<rows, kRowsThreads, 0, stream>>>(x, nb, plan.tiles == 0 ? 1 : 0,
                                                     static_cast<u32x4*>(scratch.base), factor);
@@ -581,7 +810,7 @@ hipError_t launch_q4_rows_argmax(const float* x, const Q4Mat& w, int n_blocks, f
     p.records = records;
     hipError_t e = launch_rows<kRowsArgmax>(p, x + (int64_t)r * n_blocks * 32, scratch, stream);
     const int wg_cols = 16 * rows_plan(w.n, n_blocks, p.rows).cols;  // one record each
-    const int per_row = (w.n + wg_cols - 1) / wg_cols;
+    const int per_row = pick_wide(w.n, n_blocks, p.rows) ? pick_records(p.rows) : (w.n + wg_cols - 1) / wg_cols;
     if (e == hipSuccess) e = launch_argmax_merge(records, per_row, w.n, out + r, p.rows, stream);
     if (e != hipSuccess) return e;
   }

@@ -172,7 +172,8 @@ def test_qkv_rows(H, Hkv, q, Dh, B):
             assert np.all(np.delete(c[b], row, axis=1) == np.float16(canary)), b
 
 
-@pytest.mark.parametrize("n,n_blocks,rows", [(20011, 98, 4), (20011, 98, 16), (16384, 97, 20), (33000, 33, 70)])
+@pytest.mark.parametrize("n,n_blocks,rows", [(20011, 98, 4), (20011, 98, 16), (16384, 97, 20), (33000, 33, 70),
+                                                (20017, 104, 48), (17001, 8, 48), (20480, 105, 9)])
 def test_lm_head_rows(n, n_blocks, rows):
     say(f"lm_head rows n={n} n_blocks={n_blocks} rows={rows}")
     g = rng(970 + rows)
