@@ -357,6 +357,10 @@ __global__ __launch_bounds__(kWaves * 64, kTiles == 4 ? 2 : 4) void q4_product_k
         for (int i = 0; i < 8; ++i) {
           block(a[i % kHeld], blk + i, z, i);
           load_a(a[i % kHeld], blk + i + kHeld);
+          // One block at a time: with the next ones' reads hoisted, the 64-
+          // row forms spilled (K = 3136, 5120 columns, 512 rows: 108.7 us
+          // against 73.0).
+          __builtin_amdgcn_sched_barrier(0);
         }
       } else {
 #pragma unroll
