@@ -137,6 +137,27 @@ int auto_splits(int n_heads, int n_kv_heads, int batch, int max_len) {
   }
   int n = (kTargetWorkgroups + per_wave - 1) / per_wave;              // fill the chip
   const int by_len = (max_len + kMaxKeysPerSplit - 1) / kMaxKeysPerSplit;  // bound per-split work
+  // Between half a wave and a whole one, two splits make a second wave that
+  // is nearly empty at the low end, and cost records at every length. Up to
+  // 2048 keys one split wins where a workgroup serves several heads; past
+  // that, and for single heads, splits of about 512 keys, up to 8, even the
+  // waves out where the splits so far leave a quarter of theirs idle. us per
+  // call, this against the two splits (4 at 8000 keys) before, equal lengths
+  // / lengths from an eighth up: 32q/8kv/d128, batch 17, 300 keys 8.2 / 7.6
+  // against 11.4 / 10.8, 1800 24.6 / 23.2 against 31.5 / 26.8, 4000 47.9 /
+  // 35.0 against 64.3 / 50.5, 8000 95.1 / 65.9 against 106.6 / 69.2; batch
+  // 30, 1800 keys 34.9 / 26.3 against 37.5 / 26.5; 16q/8kv/d256, batch 20,
+  // 2500 72.8 / 48.0 against 78.0 / 61.6; 32q/32kv/d96, batch 6, 1500 22.5 /
+  // 18.2 against 23.7 / 19.4; 32q/8kv/d64, batch 22, 2500 22.9 / 20.0 against
+  // 24.7 / 19.5. Where the waves were full it lost: 32q/8kv, batch 27, 2500
+  // keys 47.9 against 47.0, batch 31, 4000 85.7 against 84.2.
+  if (per_wave < kTargetWorkgroups) {
+    if (n_heads > n_kv_heads && max_len <= 2048) return 1;
+    const int64_t wgs = (int64_t)per_wave * (by_len > n ? by_len : n);
+    const int64_t waves = (wgs + kTargetWorkgroups - 1) / kTargetWorkgroups;
+    const int by_wave = (max_len + 511) / 512 < 8 ? (max_len + 511) / 512 : 8;
+    if (4 * wgs <= 3 * kTargetWorkgroups * waves && by_wave > n) n = by_wave;
+  }
   if (by_len > n) n = by_len;
   return n < 1 ? 1 : n;
 }
