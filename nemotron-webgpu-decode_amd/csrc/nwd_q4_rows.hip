@@ -59,9 +59,12 @@ struct RowsArgs {
 
 enum RowsKind { kRowsPlain = 0, kRowsQkv = 1, kRowsArgmax = 2 };
 
-// Added to a byte offset, takes a read past its descriptor's range: it
-// returns zeros without a memory access.
-constexpr int kNoRead = 0x7FFFFFFF;
+// Lane offset of a read that is not to happen: at or past every descriptor's
+// byte count (below 2^31), it returns zeros without a memory access. Only the
+// lane offset is compared with the byte count as it stands: the range check
+// subtracts the scalar offset from the count first, so a scalar offset stays
+// inside the buffer whatever the lane offset is.
+constexpr uint32_t kNoRead = 0x80000000u;
 
 // The matrix that columns col0 .. col0 + 15 lie in (a 16-column tile never
 // straddles two of them: their widths are multiples of 16), col0 made
@@ -279,6 +282,7 @@ __global__ __launch_bounds__(kWaves * 64, kTiles == 4 ? 2 : 4) void q4_product_k
 
   // ---- row groups
   const int first = wave * nb / kWaves, end = (wave + 1) * nb / kWaves;
+  const int last = max(end - 1, 0);  // requests past the part's blocks repeat its last one's
   const int groups = (p.rows + kRows * kMt - 1) / (kRows * kMt);
   const int cell0 = (lane & 15) * stride, g = (lane >> 4) & 3;
   bool staged = false;
@@ -287,13 +291,13 @@ __global__ __launch_bounds__(kWaves * 64, kTiles == 4 ? 2 : 4) void q4_product_k
         const_cast<u32x4*>(p.a + (int64_t)group * kMt * nb * kParts * 64), 0, kMt * nb * kParts * 1024, kBufferWord3);
     f16x8 a[kHeld][kMt][kParts];
     const auto load_a = [&](f16x8 (&dst)[kMt][kParts], int blk) __attribute__((always_inline)) {
-      const int off = blk < end ? 0 : kNoRead;
+      const int b = min(blk, last);
 #pragma unroll
       for (int mt = 0; mt < kMt; ++mt)
 #pragma unroll
         for (int part = 0; part < kParts; ++part)
           dst[mt][part] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(
-              ra, lane * 16, ((mt * nb + blk) * kParts + part) * 1024 | off, 0));
+              ra, lane * 16, ((mt * nb + b) * kParts + part) * 1024, 0));
     };
     f32x4 acc[kMt][kCols];
 #pragma unroll
@@ -306,7 +310,7 @@ __global__ __launch_bounds__(kWaves * 64, kTiles == 4 ? 2 : 4) void q4_product_k
 #pragma unroll
       for (int c = 0; c < kCols; ++c)
         dst[c] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(
-            rz[c], min((zcell[c] + blk) >> 1, zlast[c]), blk < end ? 0 : kNoRead, 0));
+            rz[c], min((zcell[c] + blk) >> 1, zlast[c]), 0, 0));
     };
     const auto nibbles = [&](const u32x2& v, int c, int blk) __attribute__((always_inline)) {
       const int byte = (zcell[c] + blk) >> 1;
@@ -472,16 +476,15 @@ __global__ __launch_bounds__(kPickThreads) __attribute__((amdgpu_waves_per_eu(2,
   // group's requests do not fit the memory path's queues at once: issued
   // together they held the wavefronts up for as long as the products take.
   const auto load_w = [&](int group, int first_i) __attribute__((always_inline)) {
-    const int base = group * cells;  // past the last column: out of range, zeros
-    const int off = group < groups ? 0 : kNoRead;
+    const int base = group * cells;  // past the last column: no read
 #pragma unroll
     for (int i = first_i; i < first_i + 2; ++i) {
       if (i >= kPickLoads) break;
       const int cell = base + tid + i * kPickThreads;
       const bool in = to[i] >= 0 && cell < n_cells;
       wq[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-          rq, in ? cell * 16 : kNoRead, off, kStreamPolicy));
-      ws[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, in ? cell * 4 : kNoRead, off, 0));
+          rq, in ? cell * 16 : kNoRead, 0, kStreamPolicy));
+      ws[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, in ? cell * 4 : kNoRead, 0, 0));
     }
     if (first_i + 2 < kPickLoads) return;
 #pragma unroll
@@ -490,7 +493,7 @@ __global__ __launch_bounds__(kPickThreads) __attribute__((amdgpu_waves_per_eu(2,
       for (int h = 0; h < 2; ++h) {
         const int cell = min(group * kPickCols + c * 16 + (lane & 15), m.n - 1) * nb + first + 8 * h;
         zn[c][h] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(
-            rz, min(cell >> 1, zlast), first + 8 * h < end ? off : kNoRead, 0));
+            rz, group < groups && first + 8 * h < end ? min(cell >> 1, zlast) : kNoRead, 0, 0));
       }
   };
   const auto load_all = [&](int group) __attribute__((always_inline)) {
@@ -525,7 +528,7 @@ __global__ __launch_bounds__(kPickThreads) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
     for (int part = 0; part < kParts; ++part)
       a[b][part] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(
-          ra, lane * 16, first + b < end ? ((first + b) * kParts + part) * 1024 : kNoRead, 0));
+          ra, first + b < end ? lane * 16 : kNoRead, first + b < end ? ((first + b) * kParts + part) * 1024 : 0, 0));
   // The thread's logit of a group: row tid / 32 of the tile, column tid % 32.
   const int r = tid / kPickCols, cc = tid % kPickCols, row = tile * kRows + r;
   const bool live_row = r < kRows && row < p.rows;
