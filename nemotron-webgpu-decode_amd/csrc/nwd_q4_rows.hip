@@ -8,14 +8,22 @@
 //   B  the exact integers nib - zp of one block of 16 columns, in fp16;
 //   A  16 activation rows, each scaled by a power of two so that its largest
 //      magnitude lies in [2^14, 2^15) and carried as fp16 high and low parts
-//      (hi = fp16(x), lo = fp16(x - hi): 22 to 23 bits of x), two MFMAs onto
-//      one accumulator;
+//      (hi = fp16(x), lo = fp16(x - hi)), two MFMAs onto one accumulator;
 //   D  the block's sums, multiplied by the block's scale into fp32 sums.
 // At the end a row's sums are multiplied by its power of two. Against 64 bits
 // the results are closer than those of the one-row kernels (2-norm of the
 // error over the result, K = 3136 and 5120: 1.1e-7 and 1.2e-7 against 2.2e-7
 // and 2.5e-7): the products are exact, and the zero points come off the
 // weights exactly instead of as a difference of two large sums.
+//
+// The parts hold x within 2^-23 of its magnitude, and never closer than 2^-25
+// after the scaling, where the low part is at the end of fp16's range. A row
+// with a block whose largest magnitude is more than 15 binades below the
+// row's (an activation of 10^6 beside ordinary ones) would lose bits there
+// that a weight of zero at the large element brings to light: such a row is
+// "wide", and its sums are taken in fp32 from the activations themselves, by
+// the same wavefronts over the weights in LDS (wide_dot). So every x is held
+// within 2^-23 of the largest magnitude of its block, at least.
 //
 // Two launches per call: q4_rows_kernel converts the activation rows into
 // the A operands' lane order in the context's workspace, q4_product_kernel
@@ -40,8 +48,9 @@ struct RowsArgs {
   int cols;               // all columns
   int n_blocks;
   int rows;               // activation rows of this launch
+  const float* x;         // activations [rows][32 n_blocks]
   const u32x4* a;         // A operands (q4_rows_kernel)
-  const float* factor;    // [rows] power of two of each row
+  const float* factor;    // [rows] power of two of each row (kWideRow, NaN)
   // where the results go
   int epilogue;           // Q4Epilogue (plain projections)
   float* y;               // [rows][cols]
@@ -54,6 +63,8 @@ struct RowsArgs {
   int* status;
   unsigned long long* records;  // greedy pick
   int per_row;
+  unsigned long long* wide_best;  // [rows] picks of wide rows, and the arrivals
+  int* wide_tickets;              // (q4_pick_merge_kernel); zeros from q4_rows_kernel
   int red_offset;  // of the workgroup's sums in LDS
 };
 
@@ -157,19 +168,24 @@ __device__ inline void put(const RowsArgs& p, int row, int col, float v) {
 // rows), [block] with the high parts as rows 0-7 and the low parts as rows
 // 8-15, one MFMA for both.
 // A row that holds an infinity or a NaN gets the factor NaN: the one-row
-// kernels' sums (nib x - zp x per block) give NaN for such a row too.
+// kernels' sums (nib x - zp x per block) give NaN for such a row too. A wide
+// row gets the factor kWideRow, which no power of two here is.
 constexpr int kRowsThreads = 256;
+constexpr float kWideRow = 0.f;
+constexpr uint32_t kWideBinades = 15;  // a block's largest is then at least 2^-1, the parts' step 2^-24
 constexpr int kRowsRuns = kQ4MaxBlocks * 4 / kRowsThreads;  // 8-element runs per thread
 
 __global__ __launch_bounds__(kRowsThreads) void q4_rows_kernel(const float* __restrict__ x,
                                                                int n_blocks, int packed,
                                                                u32x4* __restrict__ a,
-                                                               float* __restrict__ factor) {
-  __shared__ uint32_t wave_max[kRowsThreads / 64];
+                                                               float* __restrict__ factor,
+                                                               unsigned long long* __restrict__ wide_best,
+                                                               int* __restrict__ wide_tickets) {
+  __shared__ uint32_t wave_max[kRowsThreads / 64], wave_low[kRowsThreads / 64];
   const int row = blockIdx.x, t = threadIdx.x, runs = n_blocks * 4;
   const f32x4* xr = reinterpret_cast<const f32x4*>(x + (int64_t)row * n_blocks * 32);
   f32x4 v[kRowsRuns][2];
-  uint32_t m = 0;
+  uint32_t m = 0, low = 0xFFFFFFFFu;  // largest magnitudes: of the row, and of its smallest block not all zeros
 #pragma unroll
   for (int j = 0; j < kRowsRuns; ++j) {
     const int i = t + j * kRowsThreads;
@@ -180,24 +196,43 @@ __global__ __launch_bounds__(kRowsThreads) void q4_rows_kernel(const float* __re
   }
 #pragma unroll
   for (int j = 0; j < kRowsRuns; ++j) {
-    if (t + j * kRowsThreads < runs) {
+    if (t + j * kRowsThreads < runs) {  // the same in the 4 lanes of a block
+      uint32_t b = 0;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) m = max(m, __float_as_uint(v[j][e >> 2][e & 3]) & 0x7FFFFFFFu);
+      for (int e = 0; e < 8; ++e) b = max(b, __float_as_uint(v[j][e >> 2][e & 3]) & 0x7FFFFFFFu);
+      b = max(b, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b, kDppQuadXor1, 0xF, 0xF, false));
+      b = max(b, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b, kDppQuadXor2, 0xF, 0xF, false));
+      m = max(m, b);
+      low = min(low, b - 1u);  // zeros wrap to the top
     }
   }
 #pragma unroll
-  for (int s = 32; s >= 1; s >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, s, 64));
-  if ((t & 63) == 0) wave_max[t >> 6] = m;
+  for (int s = 32; s >= 4; s >>= 1) {
+    m = max(m, (uint32_t)__shfl_xor((int)m, s, 64));
+    low = min(low, (uint32_t)__shfl_xor((int)low, s, 64));
+  }
+  if ((t & 63) == 0) {
+    wave_max[t >> 6] = m;
+    wave_low[t >> 6] = low;
+  }
   __syncthreads();
 #pragma unroll
-  for (int w = 0; w < kRowsThreads / 64; ++w) m = max(m, wave_max[w]);
+  for (int w = 0; w < kRowsThreads / 64; ++w) {
+    m = max(m, wave_max[w]);
+    low = min(low, wave_low[w]);
+  }
   // 2^e brings the largest magnitude's exponent to 14; e stays where 2^e and
   // 2^-e are normal numbers.
   const bool finite = m < 0x7F800000u;
+  const bool wide = m != 0 && (m >> 23) - ((low + 1u) >> 23) > kWideBinades;
   const int e = min(141 - (int)(m >> 23), 126);
   const float up = finite ? __uint_as_float((uint32_t)(e + 127) << 23) : 0.f;
-  if (t == 0)
-    factor[row] = finite ? __uint_as_float((uint32_t)(127 - e) << 23) : __uint_as_float(0x7FC00000u);
+  if (t == 0) {
+    wide_best[row] = 0ull;
+    if (row == 0) *wide_tickets = 0;
+    factor[row] = !finite ? __uint_as_float(0x7FC00000u)
+                          : (wide ? kWideRow : __uint_as_float((uint32_t)(127 - e) << 23));
+  }
 #pragma unroll
   for (int j = 0; j < kRowsRuns; ++j) {
     const int i = t + j * kRowsThreads;
@@ -221,6 +256,70 @@ __global__ __launch_bounds__(kRowsThreads) void q4_rows_kernel(const float* __re
       o[0] = __builtin_bit_cast(u32x4, hi);
       o[64] = __builtin_bit_cast(u32x4, lo);
     }
+  }
+}
+
+// The factor of a row's sums: a wide row's are not scaled.
+__device__ inline float sum_factor(float factor) { return factor == kWideRow ? 1.f : factor; }
+
+// Lane l's factor of row row0 + l, of n <= 64 rows.
+__device__ inline float lane_factor(const RowsArgs& p, int row0, int n) {
+  const int lane = threadIdx.x & 63;
+  return lane < n && row0 + lane < p.rows ? p.factor[row0 + lane] : 1.f;
+}
+
+// One block of a wide row: its 32 activations times the weights less their
+// zero point, which are exact in fp16.
+__device__ inline float wide_dot(const f32x4* __restrict__ x, u32x4 q, uint32_t z) {
+  float d = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const f16x8 b = unpack(q[w], z);
+    const f32x4 v[2] = {x[2 * w], x[2 * w + 1]};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int src = (k >> 1) + (k & 1) * 4;  // 0, 4, 1, 5, 2, 6, 3, 7
+      d = fmaf((float)b[k], v[src >> 2][src & 3], d);
+    }
+  }
+  return d;
+}
+
+// The sums of the wide rows among a wavefront's, in place of its products'.
+// Lane (column l % 16, quarter l / 16) holds sums acc[mt][c][r] of row
+// 16 mt + 4 (l / 16) + r (packed: rows 8 up hold the low parts' sums, here
+// zeros). The four quarters share a row's blocks; block(c, blk, x) is the
+// lane's column's block blk of column tile c. K = 3136, 7168 columns, 16 rows:
+// 11.0 us, with one wide row 14.6, with 16 71 (one-row kernels 55).
+template <int kMt, int kCols, bool kPacked, typename Block>
+__device__ inline void wide_sums(const RowsArgs& p, uint64_t wide, int row0, int first, int end,
+                                 f32x4 (&acc)[kMt][kCols], const Block& block) {
+  const int quarter = (threadIdx.x >> 4) & 3;
+  while (wide) {
+    const int at = __builtin_ctzll(wide);
+    wide &= wide - 1;
+    const f32x4* x = reinterpret_cast<const f32x4*>(p.x + (int64_t)(row0 + at) * p.n_blocks * 32);
+    float sum[kCols];
+#pragma unroll
+    for (int c = 0; c < kCols; ++c) sum[c] = 0.f;
+#pragma unroll 1
+    for (int blk = first + quarter; blk < end; blk += 4) {
+#pragma unroll
+      for (int c = 0; c < kCols; ++c) sum[c] += block(c, blk, x + 8 * blk);
+    }
+#pragma unroll
+    for (int c = 0; c < kCols; ++c) sum[c] = sum_xor32(sum_xor16(sum[c]));
+#pragma unroll
+    for (int mt = 0; mt < kMt; ++mt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (at >> 4 == mt && (at & 3) == r) {
+#pragma unroll
+          for (int c = 0; c < kCols; ++c) {
+            if (quarter == ((at >> 2) & 3)) acc[mt][c][r] = sum[c];
+            if (kPacked && quarter == ((at >> 2) & 3) + 2) acc[mt][c][r] = 0.f;
+          }
+        }
   }
 }
 
@@ -375,6 +474,15 @@ __global__ __launch_bounds__(kWaves * 64, kTiles == 4 ? 2 : 4) void q4_product_k
       }
     }
 
+    const float factors = lane_factor(p, group * kMt * kRows, kMt * kRows);
+    const uint64_t wide = __ballot(factors == kWideRow);
+    if (wide)
+      wide_sums<kMt, kCols, !kTiles>(p, wide, group * kMt * kRows, first, end, acc, [&](int c, int blk, const f32x4* x) __attribute__((always_inline)) {
+        const int cell = c * cells + cell0 + blk, zat = zcell[c] + blk;
+        const uint32_t z = __builtin_amdgcn_raw_buffer_load_b8(rz[c], zat >> 1, 0, 0) >> (4 * (zat & 1)) & 15u;
+        return lds_s[cell] * wide_dot(x, lds_q[cell], z);
+      });
+
     // The wavefronts' sums, added in wavefront order, one row tile at a time.
 #pragma unroll
     for (int mt = 0; mt < kMt; ++mt) {
@@ -398,7 +506,7 @@ __global__ __launch_bounds__(kWaves * 64, kTiles == 4 ? 2 : 4) void q4_product_k
             if constexpr (!kTiles) v += red[(k * 16 + r + 8) * (kWgCols + kRedPad) + cc];
           }
         }
-        if (live) v *= p.factor[row];
+        v *= sum_factor(__shfl(factors, mt * kRows + (r < kRows ? r : 0), 64));
         if constexpr (kKind == kRowsArgmax) {  // one record per row and workgroup
           if (live && p.y) p.y[(int64_t)row * p.cols + cl] = v;
           unsigned long long best = live ? argmax_enc(v, cl, argmax_shape(p.cols)) : 0ull;
@@ -611,6 +719,84 @@ __global__ __launch_bounds__(kPickThreads) __attribute__((amdgpu_waves_per_eu(2,
   if (cc == 0 && live_row) p.records[(int64_t)row * p.per_row + slot] = best;
 }
 
+// The picks of q4_pick_kernel's records, a workgroup per row; and the wide
+// rows, whose logits and records there are void: all workgroups share their
+// columns out, 16 lanes to a column, and the last to arrive writes the picks.
+// (In q4_pick_kernel, code for them in its walk or after it cost every call
+// 3 to 5%.) 131072 x 3136, 16 rows: 78 us, with one wide row 158, with 16 931
+// (one-row kernels 592).
+constexpr int kPickMergeGrid = 512;
+constexpr int kPickMergeThreads = 256;
+constexpr int kWideLanes = 16;
+constexpr int kWideIters = (kPickMaxBlocks + kWideLanes - 1) / kWideLanes;
+constexpr int kWideStride = 36;  // floats of an activation block in LDS: 16 lanes' reads on distinct banks
+
+__global__ __launch_bounds__(kPickMergeThreads) void q4_pick_merge_kernel(const RowsArgs p,
+                                                                          uint32_t* __restrict__ out) {
+  __shared__ __attribute__((aligned(16))) float x[kPickMaxBlocks * kWideStride];
+  __shared__ unsigned long long best;
+  __shared__ int last;
+  const int tid = threadIdx.x, nb = p.n_blocks;
+  const ArgmaxShape shape = argmax_shape(p.cols);
+  uint64_t wide = __ballot(lane_factor(p, 0, p.rows) == kWideRow);  // at most 48 rows
+  if ((int)blockIdx.x < p.rows && !((wide >> blockIdx.x) & 1)) {
+    if (tid == 0) best = 0ull;
+    __syncthreads();
+    const unsigned long long e = wave_max_u64(tid < p.per_row ? p.records[(int64_t)blockIdx.x * p.per_row + tid] : 0ull);
+    if ((tid & 63) == 0) atomicMax(&best, e);
+    __syncthreads();
+    if (tid == 0) out[blockIdx.x] = argmax_decode(best, shape);
+  }
+  if (!wide) return;
+  const Q4Mat m = p.m[0];
+  const int part = tid % kWideLanes, group = tid / kWideLanes;
+  for (uint64_t left = wide; left; left &= left - 1) {
+    const int row = __builtin_ctzll(left);
+    const float* xr = p.x + (int64_t)row * nb * 32;
+    __syncthreads();
+    if (tid == 0) best = 0ull;
+    for (int i = tid; i < nb * 32; i += kPickMergeThreads) x[i / 32 * kWideStride + i % 32] = xr[i];
+    __syncthreads();
+    unsigned long long e = 0ull;
+    for (int col = blockIdx.x * (kPickMergeThreads / kWideLanes) + group; col < p.cols;
+         col += gridDim.x * (kPickMergeThreads / kWideLanes)) {
+      u32x4 q[kWideIters];
+      float s[kWideIters];
+      uint32_t z[kWideIters];
+#pragma unroll
+      for (int i = 0; i < kWideIters; ++i) {  // past the last block: its weights again, times zero
+        const int blk = part + i * kWideLanes;
+        const int64_t cell = (int64_t)col * nb + min(blk, nb - 1);
+        q[i] = *reinterpret_cast<const u32x4*>(m.quant + cell * 16);
+        s[i] = m.scales[cell];
+        z[i] = m.zp[cell >> 1] >> (4 * (cell & 1)) & 15u;
+      }
+      float v = 0.f;
+#pragma unroll
+      for (int i = 0; i < kWideIters; ++i) {
+        const int blk = part + i * kWideLanes;
+        const float d = s[i] * wide_dot(reinterpret_cast<const f32x4*>(x + min(blk, nb - 1) * kWideStride), q[i], z[i]);
+        v += blk < nb ? d : 0.f;
+      }
+      v = sum8(v);
+      v += dpp_mov<kDppRowMirror>(v);
+      if (part == 0) {
+        if (p.y) p.y[(int64_t)row * p.cols + col] = v;
+        const unsigned long long c = argmax_enc(v, col, shape);
+        e = c > e ? c : e;
+      }
+    }
+    if (e) atomicMax(&best, e);
+    __syncthreads();
+    if (tid == 0) __hip_atomic_fetch_max(p.wide_best + row, best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (tid == 0)
+    last = __hip_atomic_fetch_add(p.wide_tickets, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
+  __syncthreads();
+  if (last && tid < p.rows && ((wide >> tid) & 1))
+    out[tid] = argmax_decode(__hip_atomic_load(p.wide_best + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), shape);
+}
+
 // ------------------------------------------------------------------- launch
 
 constexpr int kPackedRows = 8;
@@ -675,13 +861,14 @@ int pick_records(int rows) {
 }
 static_assert(pick_lds(kPickMaxBlocks) <= 160 * 1024, "the weights of two groups and the sums fit a CU");
 
-// Bytes of A operands and factors that `rows` rows of a launch take.
+// Scratch of `rows` rows of a launch: the A operands, then each row's factor,
+// the wide rows' picks and their tickets.
 size_t factor_offset(int rows, int n_blocks) {
   return rows <= kPackedRows ? (size_t)n_blocks * 1024 : (size_t)((rows + 63) / 64 * 4) * n_blocks * 2048;
 }
-size_t rows_bytes(int rows, int n_blocks) {
-  return factor_offset(rows, n_blocks) + (size_t)((rows + 3) / 4) * 16;
-}
+size_t best_offset(int rows, int n_blocks) { return factor_offset(rows, n_blocks) + (size_t)((rows + 3) / 4) * 16; }
+size_t tickets_offset(int rows, int n_blocks) { return best_offset(rows, n_blocks) + (size_t)((rows + 1) / 2) * 16; }
+size_t rows_bytes(int rows, int n_blocks) { return tickets_offset(rows, n_blocks) + 16; }
 
 // Rows per launch within the scratch: all of them, or a multiple of 64 or 8.
 int rows_per_launch(int rows, int n_blocks, size_t scratch) {
@@ -693,17 +880,21 @@ int rows_per_launch(int rows, int n_blocks, size_t scratch) {
 }
 
 template <int kKind>
-hipError_t launch_rows(RowsArgs p, const float* x, Q4Scratch scratch, hipStream_t stream) {
+hipError_t launch_rows(RowsArgs p, const float* x, Q4Scratch scratch, uint32_t* out, hipStream_t stream) {
   const int rows = p.rows, nb = p.n_blocks;
-  p.a = reinterpret_cast<const u32x4*>(scratch.base);
-  float* factor = reinterpret_cast<float*>(static_cast<char*>(scratch.base) + factor_offset(rows, nb));
+  p.x = x;
+  char* base = static_cast<char*>(scratch.base);
+  p.a = reinterpret_cast<const u32x4*>(base);
+  float* factor = reinterpret_cast<float*>(base + factor_offset(rows, nb));
   p.factor = factor;
+  p.wide_best = reinterpret_cast<unsigned long long*>(base + best_offset(rows, nb));
+  p.wide_tickets = reinterpret_cast<int*>(base + tickets_offset(rows, nb));
   if constexpr (kKind == kRowsArgmax) {
     if (pick_wide(p.cols, nb, rows)) {
       const bool packed = rows <= kPackedRows;
       const int tiles = packed ? 1 : (rows + 15) / 16;
-      q4_rows_kernel<<<rows, kRowsThreads, 0, stream>>>(x, nb, packed ? 1 : 0,
-                                                        static_cast<u32x4*>(scratch.base), factor);
+      q4_rows_kernel<<<rows, kRowsThreads, 0, stream>>>(x, nb, packed ? 1 : 0, reinterpret_cast<u32x4*>(base), factor,
+                                                        p.wide_best, p.wide_tickets);
       hipError_t e = hipGetLastError();
       const void* kern = packed ? reinterpret_cast<const void*>(q4_pick_kernel<0>)
                                 : reinterpret_cast<const void*>(q4_pick_kernel<1>);
@@ -715,12 +906,14 @@ hipError_t launch_rows(RowsArgs p, const float* x, Q4Scratch scratch, hipStream_
         q4_pick_kernel<0><<<tiles * p.per_row, kPickThreads, pick_lds(nb), stream>>>(p, tiles);
       else
         q4_pick_kernel<1><<<tiles * p.per_row, kPickThreads, pick_lds(nb), stream>>>(p, tiles);
+      if ((e = hipGetLastError()) != hipSuccess) return e;
+      q4_pick_merge_kernel<<<kPickMergeGrid, kPickMergeThreads, 0, stream>>>(p, out);
       return hipGetLastError();
     }
   }
   const RowsPlan plan = rows_plan(p.cols, nb, rows);
-  q4_rows_kernel<<<rows, kRowsThreads, 0, stream>>>(x, nb, plan.tiles == 0 ? 1 : 0,
-                                                    static_cast<u32x4*>(scratch.base), factor);
+  q4_rows_kernel<<<rows, kRowsThreads, 0, stream>>>(x, nb, plan.tiles == 0 ? 1 : 0, reinterpret_cast<u32x4*>(base),
+                                                    factor, p.wide_best, p.wide_tickets);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const int wg_cols = plan.cols * 16, wg_rows = plan.tiles ? 16 * plan.tiles : kPackedRows;
@@ -737,7 +930,8 @@ hipError_t launch_rows(RowsArgs p, const float* x, Q4Scratch scratch, hipStream_
                             hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);          \
     if (e != hipSuccess) return e;                                                            \
     q4_product_kernel<T, C, W, kKind><<<grid, W * 64, lds, stream>>>(p);                      \
-    return hipGetLastError();                                                                 \
+    if ((e = hipGetLastError()) != hipSuccess || kKind != kRowsArgmax) return e;              \
+    return launch_argmax_merge(p.records, p.per_row, p.cols, out, rows, stream);              \
   }
   NWD_ROWS_CASE(0, 1, 8) NWD_ROWS_CASE(0, 2, 8) NWD_ROWS_CASE(1, 1, 8) NWD_ROWS_CASE(1, 2, 8)
   NWD_ROWS_CASE(2, 1, 8) NWD_ROWS_CASE(2, 2, 8) NWD_ROWS_CASE(4, 1, 8) NWD_ROWS_CASE(4, 2, 8)
@@ -774,7 +968,7 @@ hipError_t launch_q4_rows_gemv(const float* x, const Q4Mat& w, int n_blocks, flo
     p.rows = rows - r < per ? rows - r : per;
     p.epilogue = epilogue;
     p.y = y + (int64_t)r * w.n;
-    const hipError_t e = launch_rows<kRowsPlain>(p, x + (int64_t)r * n_blocks * 32, scratch, stream);
+    const hipError_t e = launch_rows<kRowsPlain>(p, x + (int64_t)r * n_blocks * 32, scratch, nullptr, stream);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
@@ -800,7 +994,7 @@ hipError_t launch_q4_rows_qkv(const Shape& s, const float* x, const Q4Mat& wq, c
     p.q16 = s.q16;
     p.cache_size = p.rows * seq;
     p.status = status;
-    const hipError_t e = launch_rows<kRowsQkv>(p, x + (int64_t)r * n_blocks * 32, scratch, stream);
+    const hipError_t e = launch_rows<kRowsQkv>(p, x + (int64_t)r * n_blocks * 32, scratch, nullptr, stream);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
@@ -815,10 +1009,7 @@ hipError_t launch_q4_rows_argmax(const float* x, const Q4Mat& w, int n_blocks, f
     p.rows = batch - r < per ? batch - r : per;
     p.y = logits ? logits + (int64_t)r * w.n : nullptr;
     p.records = records;
-    hipError_t e = launch_rows<kRowsArgmax>(p, x + (int64_t)r * n_blocks * 32, scratch, stream);
-    const int wg_cols = 16 * rows_plan(w.n, n_blocks, p.rows).cols;  // one record each
-    const int per_row = pick_wide(w.n, n_blocks, p.rows) ? pick_records(p.rows) : (w.n + wg_cols - 1) / wg_cols;
-    if (e == hipSuccess) e = launch_argmax_merge(records, per_row, w.n, out + r, p.rows, stream);
+    const hipError_t e = launch_rows<kRowsArgmax>(p, x + (int64_t)r * n_blocks * 32, scratch, out + r, stream);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

@@ -2,10 +2,10 @@
 kernels of nwd_q4_rows.hip) with float64, through the C ABI.
 
 Bars: |y - y64| <= 1e-6 sum_k |w_k a_k| (the one-row kernels' bar; their
-activations enter as fp16 high and low parts, within 2^-22 of each, and 32
-products are summed at a time); a row that holds an infinity or a NaN is NaN,
-as on the one-row kernels; cache rows within one fp16 ulp; the picked token
-is the largest logit.
+activations enter as fp16 high and low parts, within 2^-23 of the largest of
+their 32, or in fp32, and 32 products are summed at a time); a row that holds
+an infinity or a NaN is NaN, as on the one-row kernels; cache rows within one
+fp16 ulp; the picked token is the largest logit.
 
 Sizes: the smallest and largest row counts of each row tiling (packed up to
 8, then 16, 32 and 64 rows, several groups of 64), column counts that leave a
@@ -132,6 +132,68 @@ def test_rows_ranges_and_non_finite():
     y64, bound = w.f64(x[fine])
     # a subnormal result is within half its last place, 2^-150
     assert np.all(np.abs(got[fine] - y64) <= TOL_REL * bound + 2.0 ** -149)
+
+
+def _hide_block(w, n, n_blocks, blk):
+    """Block blk of every column gets no weight: nibbles and zero point 0 in
+    even columns (the form the one-row kernels keep exact), 9 in odd ones."""
+    quant, _, zp = w.t
+    value = torch.arange(n, device="cuda") % 2 * 9
+    quant[:, blk] = (value * 17).to(torch.uint8).unsqueeze(1)
+    cell = torch.arange(n, device="cuda") * n_blocks + blk
+    for half in (0, 1):
+        at = cell % 2 == half
+        b = cell[at] // 2
+        keep = zp[b] & (0xF0 if half == 0 else 0x0F)
+        zp[b] = keep | (value[at] << (4 * half)).to(torch.uint8)
+    w.dense[:, 32 * blk:32 * blk + 32] = 0
+
+
+@pytest.mark.parametrize("n,n_blocks,rows,head", [
+    (4096, 98, 8, False),     # packed
+    (1007, 98, 16, False), (1007, 97, 32, False),
+    (3136, 160, 64, False), (5120, 98, 130, False),
+    (16400, 98, 7, True), (20011, 98, 48, True),  # wide picks
+    (16400, 105, 16, True),                       # the other kernel's
+])
+def test_wide_rows(n, n_blocks, rows, head):
+    """Rows with one activation far above the rest, in a block without
+    weight: what the others lose beside it shows, and must be no more than
+    on the one-row kernels (the even columns; those lose everything in the
+    odd ones, where the large element's products cancel)."""
+    say(f"q4 wide rows n={n} n_blocks={n_blocks} rows={rows}")
+    g = rng(953 + rows)
+    w = Q4(g, n, n_blocks)
+    blk = n_blocks // 3
+    _hide_block(w, n, n_blocks, blk)
+    x = g.standard_normal((rows, 32 * n_blocks)).astype(np.float32)
+    large = [1e4, 2e5, 1e6, 1e8, 1e20]
+    for b in range(0, rows, 2):  # ordinary rows between them
+        x[b, 32 * blk + b % 32] = large[b // 2 % len(large)]
+    x[1, :32] *= np.float32(1e-6)  # the other way about: a block far below the rest
+    y = torch.full((rows, n), float("nan"), dtype=torch.float32, device="cuda")
+    one = torch.empty_like(y)
+    token = torch.full((rows,), -1, dtype=torch.int32, device="cuda")
+    dx = dev(x)
+    with _ctx() as ctx:
+        if head:
+            ctx.lm_head_argmax(dx, w.w, token, y, rows)
+        else:
+            ctx.q4_gemv(dx, w.w, y, rows)
+        for b in range(rows):
+            ctx.q4_gemv(dx[b:b + 1], w.w, one[b:b + 1], 1)
+        got, one = host(y), host(one)
+    y64, bound = w.f64(x)  # the large elements are not in the bound
+    assert np.all(np.abs(got - y64) <= TOL_REL * bound)
+
+    def err(v):
+        return np.linalg.norm((v - y64)[:, ::2], axis=1) / np.linalg.norm(y64[:, ::2], axis=1)
+
+    # 2-norms over hundreds of columns of errors of one size: 1.25 is far
+    # outside their spread, and the parts gave 2 (at 1e6) to 10^6 times
+    assert np.all(err(got) <= 1.25 * err(one)), (err(got) / err(one)).max()
+    if head:
+        np.testing.assert_array_equal(host(token), np.argmax(got, axis=1))
 
 
 @pytest.mark.parametrize("H,Hkv,q,Dh,B", [(40, 8, "f32", 128, 3), (32, 8, "f16", 128, 12),
