@@ -15,7 +15,8 @@ from pathlib import Path
 import pytest
 
 CSRC = Path(__file__).resolve().parent.parent / "nemotron-webgpu-decode_amd" / "csrc"
-MARKER = re.compile(r"\b(kNoRead|oob|0x80000000u?|0x7FFFFFFFu?)\b", re.I)
+# (after an & the number is a mask: of a float's sign, of a nibble's place)
+MARKER = re.compile(r"(?<!& )\b(kNoRead|oob|0x80000000u?|0x7FFFFFFFu?)\b", re.I)
 LOADS = re.compile(r"__builtin_amdgcn_raw_(ptr_)?buffer_load_(\w+)\s*\(")
 
 
