@@ -776,14 +776,11 @@ static int check_q4(nwd_ctx* ctx, const char* who, const char* name, const nwd_q
   return NWD_OK;
 }
 
-// The split-K workspace past its first `used` bytes, for the activation rows
-// of a projection (calls on a context are stream-ordered, so they never
-// overlap a decode's use of it).
-static nwd::Q4Scratch q4_scratch(const nwd_ctx* ctx, size_t used) {
-  const size_t have = (size_t)ctx->o_floats * sizeof(float);
-  used = (used + 255) / 256 * 256;
-  if (used >= have) return nwd::Q4Scratch{nullptr, 0};
-  return nwd::Q4Scratch{reinterpret_cast<char*>(ctx->ws.part_o) + used, have - used};
+// The split-K workspace, for the activation rows and the pick records of a
+// projection (calls on a context are stream-ordered, so they never overlap a
+// decode's use of it).
+static nwd::Q4Scratch q4_scratch(const nwd_ctx* ctx) {
+  return nwd::Q4Scratch{ctx->ws.part_o, (size_t)ctx->o_floats * sizeof(float)};
 }
 
 static nwd::Q4Mat q4_mat(const nwd_q4_weight* w) {
@@ -804,7 +801,7 @@ int nwd_q4_gemv(nwd_ctx* ctx, const float* a, const nwd_q4_weight* w, float* y, 
   if (epilogue != NWD_Q4_PLAIN && epilogue != NWD_Q4_RELU2 && epilogue != NWD_Q4_ACCUMULATE)
     return fail(ctx, NWD_ERR_INVALID, "%s: unknown epilogue %d", who, epilogue);
   hipError_t e = nwd::launch_q4_gemv(a, q4_mat(w), w->n_blocks, y, batch, epilogue,
-                                     q4_scratch(ctx, 0), (hipStream_t)stream);
+                                     q4_scratch(ctx), (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(ctx, "nwd_q4_gemv: launch", e);
   return NWD_OK;
 }
@@ -838,7 +835,7 @@ int nwd_qkv_append(nwd_ctx* ctx, const float* x, const nwd_q4_weight* wq, const 
                 ctx->desc.max_batch);
   hipError_t e = nwd::launch_qkv_append(ctx->shape, x, q4_mat(wq), q4_mat(wk), q4_mat(wv),
                                         wq->n_blocks, q_out, k_cache, v_cache, pos, batch,
-                                        ctx->ws.status, q4_scratch(ctx, 0), (hipStream_t)stream);
+                                        ctx->ws.status, q4_scratch(ctx), (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(ctx, "nwd_qkv_append: launch", e);
   return NWD_OK;
 }
@@ -884,11 +881,11 @@ int nwd_lm_head_argmax(nwd_ctx* ctx, const float* h, const nwd_q4_weight* w, flo
   if (batch < 1 || batch > 65535)
     return fail(ctx, NWD_ERR_INVALID, "%s: batch %d outside [1, 65535]", who, batch);
   int rc;
-  const int64_t n_rec = (int64_t)nwd::q4_argmax_records_per_row(w->n) * batch;
-  unsigned long long* rec = argmax_records(ctx, who, n_rec, &rc);
-  if (!rec) return rc;
-  hipError_t e = nwd::launch_q4_argmax(h, q4_mat(w), w->n_blocks, logits, out, batch, rec,
-                                       q4_scratch(ctx, (size_t)n_rec * 8), (hipStream_t)stream);
+  // The one-row kernels' records bound the batch; those of several rows need
+  // fewer, and share the workspace with their activations.
+  if (!argmax_records(ctx, who, (int64_t)nwd::q4_argmax_records_per_row(w->n) * batch, &rc)) return rc;
+  hipError_t e = nwd::launch_q4_argmax(h, q4_mat(w), w->n_blocks, logits, out, batch,
+                                       q4_scratch(ctx), (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(ctx, "nwd_lm_head_argmax: launch", e);
   return NWD_OK;
 }

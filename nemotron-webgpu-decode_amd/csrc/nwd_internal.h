@@ -192,8 +192,7 @@ hipError_t launch_q4_rows_qkv(const Shape& s, const float* x, const Q4Mat& wq, c
                               void* v_cache, const int32_t* pos, int batch, int* status,
                               Q4Scratch scratch, hipStream_t stream);
 hipError_t launch_q4_rows_argmax(const float* x, const Q4Mat& w, int n_blocks, float* logits,
-                                 uint32_t* out, int batch, unsigned long long* records,
-                                 Q4Scratch scratch, hipStream_t stream);
+                                 uint32_t* out, int batch, Q4Scratch scratch, hipStream_t stream);
 
 // y[b][n] = epilogue(dequant(W) . x[b]) for b < batch; x [batch][K] f32.
 hipError_t launch_q4_gemv(const float* x, const Q4Mat& w, int n_blocks, float* y, int batch,
@@ -223,7 +222,6 @@ hipError_t launch_argmax_merge(const unsigned long long* records, int per_row, i
 // q4_argmax_records_per_row(w.n) * batch entries.
 int q4_argmax_records_per_row(int n);
 hipError_t launch_q4_argmax(const float* x, const Q4Mat& w, int n_blocks, float* logits,
-                            uint32_t* out, int batch, unsigned long long* records,
-                            Q4Scratch scratch, hipStream_t stream);
+                            uint32_t* out, int batch, Q4Scratch scratch, hipStream_t stream);
 
 }  // namespace nwd

@@ -562,10 +562,10 @@ hipError_t launch_q4_gemv(const float* x, const Q4Mat& w, int n_blocks, float* y
 int q4_argmax_records_per_row(int n) { return (n + kQ4WgCols - 1) / kQ4WgCols; }
 
 hipError_t launch_q4_argmax(const float* x, const Q4Mat& w, int n_blocks, float* logits,
-                            uint32_t* out, int batch, unsigned long long* records,
-                            Q4Scratch scratch, hipStream_t stream) {
+                            uint32_t* out, int batch, Q4Scratch scratch, hipStream_t stream) {
   if (q4_rows_shape(w.n, w.n, n_blocks, batch, true, scratch))
-    return launch_q4_rows_argmax(x, w, n_blocks, logits, out, batch, records, scratch, stream);
+    return launch_q4_rows_argmax(x, w, n_blocks, logits, out, batch, scratch, stream);
+  unsigned long long* records = static_cast<unsigned long long*>(scratch.base);
   const int per_row = q4_argmax_records_per_row(w.n);
   const dim3 grid(per_row, batch);
   const int iters = q4w_iters(n_blocks);  // 0 past 24 blocks per lane (K > 6144)

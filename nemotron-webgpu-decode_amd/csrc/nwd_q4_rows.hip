@@ -855,44 +855,61 @@ constexpr int kPickGrid = 256;
 bool pick_wide(int cols, int n_blocks, int rows) {
   return cols >= 16384 && n_blocks <= kPickMaxBlocks && rows <= 48;
 }
-int pick_records(int rows) {
-  const int tiles = rows <= kPackedRows ? 1 : (rows + 15) / 16;
-  return kPickGrid / tiles;
+int pick_tiles(int rows) { return rows <= kPackedRows ? 1 : (rows + 15) / 16; }
+int records_per_row(int cols, int n_blocks, int rows) {
+  if (pick_wide(cols, n_blocks, rows)) return kPickGrid / pick_tiles(rows);
+  const int wg_cols = 16 * rows_plan(cols, n_blocks, rows).cols;
+  return (cols + wg_cols - 1) / wg_cols;
 }
 static_assert(pick_lds(kPickMaxBlocks) <= 160 * 1024, "the weights of two groups and the sums fit a CU");
 
-// Scratch of `rows` rows of a launch: the A operands, then each row's factor,
-// the wide rows' picks and their tickets.
-size_t factor_offset(int rows, int n_blocks) {
-  return rows <= kPackedRows ? (size_t)n_blocks * 1024 : (size_t)((rows + 63) / 64 * 4) * n_blocks * 2048;
+// Scratch of a launch: the A operands (whole row groups, which the products
+// read), each row's factor, the wide rows' picks and their tickets, and for
+// greedy picks the records, a workgroup's one per row.
+struct RowsLayout {
+  size_t factor, best, tickets, records, bytes;
+};
+RowsLayout rows_layout(int cols, int n_blocks, int rows, bool pick) {
+  const int tiles = rows <= 16 ? 1 : (rows <= 32 ? 2 : (rows + 63) / 64 * 4);
+  RowsLayout l;
+  l.factor = (size_t)n_blocks * (rows <= kPackedRows ? 1024 : tiles * (size_t)2048);
+  l.best = l.factor + (size_t)((rows + 3) / 4) * 16;
+  l.tickets = l.best + (size_t)((rows + 1) / 2) * 16;
+  l.records = l.tickets + 16;
+  l.bytes = l.records;
+  if (pick) l.bytes += (size_t)rows * records_per_row(cols, n_blocks, rows) * 8;
+  return l;
 }
-size_t best_offset(int rows, int n_blocks) { return factor_offset(rows, n_blocks) + (size_t)((rows + 3) / 4) * 16; }
-size_t tickets_offset(int rows, int n_blocks) { return best_offset(rows, n_blocks) + (size_t)((rows + 1) / 2) * 16; }
-size_t rows_bytes(int rows, int n_blocks) { return tickets_offset(rows, n_blocks) + 16; }
 
-// Rows per launch within the scratch: all of them, or a multiple of 64 or 8.
-int rows_per_launch(int rows, int n_blocks, size_t scratch) {
-  if (rows_bytes(rows, n_blocks) <= scratch) return rows;
-  int r = rows / 64 * 64;
-  while (r > 64 && rows_bytes(r, n_blocks) > scratch) r -= 64;
-  if (r >= 64 && rows_bytes(r, n_blocks) <= scratch) return r;
-  return rows_bytes(kPackedRows, n_blocks) <= scratch ? kPackedRows : 0;
+// Rows per launch within the scratch: all of them, a multiple of 64, or what
+// fewer row tiles hold.
+int rows_per_launch(int cols, int n_blocks, int rows, bool pick, size_t scratch) {
+  const auto fits = [&](int r) { return rows_layout(cols, n_blocks, r, pick).bytes <= scratch; };
+  if (fits(rows)) return rows;
+  for (int r = (rows - 1) / 64 * 64; r >= 64; r -= 64)
+    if (fits(r)) return r;
+  for (int r : {32, 16, kPackedRows})
+    if (r < rows && fits(r)) return r;
+  return 0;
 }
 
 template <int kKind>
 hipError_t launch_rows(RowsArgs p, const float* x, Q4Scratch scratch, uint32_t* out, hipStream_t stream) {
   const int rows = p.rows, nb = p.n_blocks;
   p.x = x;
+  const RowsLayout at = rows_layout(p.cols, nb, rows, kKind == kRowsArgmax);
   char* base = static_cast<char*>(scratch.base);
   p.a = reinterpret_cast<const u32x4*>(base);
-  float* factor = reinterpret_cast<float*>(base + factor_offset(rows, nb));
+  float* factor = reinterpret_cast<float*>(base + at.factor);
   p.factor = factor;
-  p.wide_best = reinterpret_cast<unsigned long long*>(base + best_offset(rows, nb));
-  p.wide_tickets = reinterpret_cast<int*>(base + tickets_offset(rows, nb));
+  p.wide_best = reinterpret_cast<unsigned long long*>(base + at.best);
+  p.wide_tickets = reinterpret_cast<int*>(base + at.tickets);
+  p.records = reinterpret_cast<unsigned long long*>(base + at.records);
+  p.per_row = kKind == kRowsArgmax ? records_per_row(p.cols, nb, rows) : 0;
   if constexpr (kKind == kRowsArgmax) {
     if (pick_wide(p.cols, nb, rows)) {
       const bool packed = rows <= kPackedRows;
-      const int tiles = packed ? 1 : (rows + 15) / 16;
+      const int tiles = pick_tiles(rows);
       q4_rows_kernel<<<rows, kRowsThreads, 0, stream>>>(x, nb, packed ? 1 : 0, reinterpret_cast<u32x4*>(base), factor,
                                                         p.wide_best, p.wide_tickets);
       hipError_t e = hipGetLastError();
@@ -901,7 +918,6 @@ hipError_t launch_rows(RowsArgs p, const float* x, Q4Scratch scratch, uint32_t* 
       if (e == hipSuccess)
         e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
       if (e != hipSuccess) return e;
-      p.per_row = pick_records(rows);
       if (packed)
         q4_pick_kernel<0><<<tiles * p.per_row, kPickThreads, pick_lds(nb), stream>>>(p, tiles);
       else
@@ -919,7 +935,6 @@ hipError_t launch_rows(RowsArgs p, const float* x, Q4Scratch scratch, uint32_t* 
   const int wg_cols = plan.cols * 16, wg_rows = plan.tiles ? 16 * plan.tiles : kPackedRows;
   const int groups = (rows + wg_rows - 1) / wg_rows, split = groups < plan.split ? groups : plan.split;
   const dim3 grid((p.cols + wg_cols - 1) / wg_cols, split);
-  p.per_row = grid.x;
   // The sums may overwrite the weights where no other row group follows.
   const int weights = plan.cols * tile_cells(nb) * kCellBytes, sums = red_floats(plan.waves, plan.cols) * 4;
   p.red_offset = split == groups ? 0 : weights;
@@ -957,12 +972,12 @@ bool q4_rows_shape(int n, int narrowest, int n_blocks, int rows, bool pick, Q4Sc
   const int64_t cells = (int64_t)n * n_blocks;
   return rows >= 2 && cells * rows >= (pick && n >= 16384 ? 6000000 : 1500000) &&
          (int64_t)narrowest * n_blocks >= 16 && cells * 16 < ((int64_t)1 << 31) - (1 << 20) &&
-         rows_per_launch(rows, n_blocks, scratch.bytes) > 0;
+         rows_per_launch(n, n_blocks, rows, pick, scratch.bytes) > 0;
 }
 
 hipError_t launch_q4_rows_gemv(const float* x, const Q4Mat& w, int n_blocks, float* y, int rows,
                                int epilogue, Q4Scratch scratch, hipStream_t stream) {
-  const int per = rows_per_launch(rows, n_blocks, scratch.bytes);
+  const int per = rows_per_launch(w.n, n_blocks, rows, false, scratch.bytes);
   for (int r = 0; r < rows; r += per) {
     RowsArgs p = rows_args(&w, 1, n_blocks);
     p.rows = rows - r < per ? rows - r : per;
@@ -979,7 +994,7 @@ hipError_t launch_q4_rows_qkv(const Shape& s, const float* x, const Q4Mat& wq, c
                               void* v_cache, const int32_t* pos, int batch, int* status,
                               Q4Scratch scratch, hipStream_t stream) {
   const Q4Mat m[3] = {wq, wk, wv};
-  const int per = rows_per_launch(batch, n_blocks, scratch.bytes);
+  const int per = rows_per_launch(wq.n + wk.n + wv.n, n_blocks, batch, false, scratch.bytes);
   const int64_t seq = (int64_t)s.n_kv * s.cap * s.head_dim;  // cache elements per sequence
   for (int r = 0; r < batch; r += per) {
     RowsArgs p = rows_args(m, 3, n_blocks);
@@ -1001,14 +1016,12 @@ hipError_t launch_q4_rows_qkv(const Shape& s, const float* x, const Q4Mat& wq, c
 }
 
 hipError_t launch_q4_rows_argmax(const float* x, const Q4Mat& w, int n_blocks, float* logits,
-                                 uint32_t* out, int batch, unsigned long long* records,
-                                 Q4Scratch scratch, hipStream_t stream) {
-  const int per = rows_per_launch(batch, n_blocks, scratch.bytes);
+                                 uint32_t* out, int batch, Q4Scratch scratch, hipStream_t stream) {
+  const int per = rows_per_launch(w.n, n_blocks, batch, true, scratch.bytes);
   for (int r = 0; r < batch; r += per) {
     RowsArgs p = rows_args(&w, 1, n_blocks);
     p.rows = batch - r < per ? batch - r : per;
     p.y = logits ? logits + (int64_t)r * w.n : nullptr;
-    p.records = records;
     const hipError_t e = launch_rows<kRowsArgmax>(p, x + (int64_t)r * n_blocks * 32, scratch, out + r, stream);
     if (e != hipSuccess) return e;
   }

@@ -251,3 +251,31 @@ def test_lm_head_rows(n, n_blocks, rows):
     assert np.all(np.abs(got - y64) <= TOL_REL * bound)
     np.testing.assert_array_equal(tok[0], np.argmax(got, axis=1))
     np.testing.assert_array_equal(tok[1], tok[0])
+
+
+def test_lm_head_fills_the_workspace():
+    """Batches up to the largest that the workspace takes (128 rows of 1024
+    records here, its 1 MiB) run the kernels of several rows as they do in a
+    roomy context: the same bits. One row more is refused."""
+    say("lm_head in a full workspace")
+    n, nb = 16384, 20
+    g = rng(980)
+    w = Q4(g, n, nb)
+    x = g.standard_normal((129, 32 * nb)).astype(np.float32)
+    dx = dev(x)
+    y64, bound = w.f64(x)
+    with _ctx(4, 4, 256, 1) as small, _ctx() as roomy:
+        for rows in (60, 100, 126, 128):
+            got, tok = [], []
+            for ctx in (small, roomy):
+                logits = torch.full((rows, n), float("nan"), dtype=torch.float32, device="cuda")
+                token = torch.full((rows,), -1, dtype=torch.int32, device="cuda")
+                ctx.lm_head_argmax(dx, w.w, token, logits, rows)
+                got.append(host(logits))
+                tok.append(host(token))
+            np.testing.assert_array_equal(got[0], got[1])
+            np.testing.assert_array_equal(tok[0], np.argmax(got[0], axis=1))
+            np.testing.assert_array_equal(tok[1], tok[0])
+            assert np.all(np.abs(got[0] - y64[:rows]) <= TOL_REL * bound[:rows])
+        with pytest.raises(nw.NwdError):
+            small.lm_head_argmax(dx, w.w, torch.empty(129, dtype=torch.int32, device="cuda"), None, 129)
