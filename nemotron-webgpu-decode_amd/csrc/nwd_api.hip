@@ -780,7 +780,7 @@ static int check_q4(nwd_ctx* ctx, const char* who, const char* name, const nwd_q
 // projection (calls on a context are stream-ordered, so they never overlap a
 // decode's use of it).
 static nwd::Q4Scratch q4_scratch(const nwd_ctx* ctx) {
-  return nwd::Q4Scratch{ctx->ws.part_o, (size_t)ctx->o_floats * sizeof(float)};
+  return nwd::Q4Scratch{ctx->ws.part_o, (size_t)ctx->o_floats * sizeof(float), ctx->ws.status};
 }
 
 static nwd::Q4Mat q4_mat(const nwd_q4_weight* w) {

@@ -42,7 +42,9 @@ constexpr int kStatusQueryRange = 4;
 
 // Bounds-checked builds (compiled with -DNWD_CHECK) check every kernel
 // store into an output, a cache or the split-K workspace, and the merges'
-// reads of the workspace: the element range [at, at + n) must lie in
+// reads of the workspace (but for the outputs and pick records of the one-row
+// 4-bit projections and of argmax, whose columns are compared with their
+// count at the store): the element range [at, at + n) must lie in
 // [0, size), the size the call's shape (or the workspace's capacity)
 // implies. An access outside it is skipped and sets kStatusOutOfBounds;
 // other builds compile the check away.

@@ -166,10 +166,12 @@ constexpr int kQ4MaxBlocks = 256;
 enum Q4Epilogue { kQ4None = 0, kQ4Relu2 = 1, kQ4Accumulate = 2 };
 
 // Workspace that a projection of several rows converts its activations into
-// (nwd_q4_rows.hip): 16-byte aligned device memory of the context.
+// (nwd_q4_rows.hip), 16-byte aligned device memory of the context, and the
+// context's status word.
 struct Q4Scratch {
   void* base;
   size_t bytes;
+  int* status;
 };
 
 // Whether the matrix-core kernels take a projection of n columns (all three
@@ -189,8 +191,8 @@ hipError_t launch_q4_rows_gemv(const float* x, const Q4Mat& w, int n_blocks, flo
                                int epilogue, Q4Scratch scratch, hipStream_t stream);
 hipError_t launch_q4_rows_qkv(const Shape& s, const float* x, const Q4Mat& wq, const Q4Mat& wk,
                               const Q4Mat& wv, int n_blocks, void* q_out, void* k_cache,
-                              void* v_cache, const int32_t* pos, int batch, int* status,
-                              Q4Scratch scratch, hipStream_t stream);
+                              void* v_cache, const int32_t* pos, int batch, Q4Scratch scratch,
+                              hipStream_t stream);
 hipError_t launch_q4_rows_argmax(const float* x, const Q4Mat& w, int n_blocks, float* logits,
                                  uint32_t* out, int batch, Q4Scratch scratch, hipStream_t stream);
 

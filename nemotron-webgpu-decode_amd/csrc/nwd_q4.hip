@@ -603,7 +603,7 @@ hipError_t launch_qkv_append(const Shape& s, const float* x, const Q4Mat& wq, co
                              Q4Scratch scratch, hipStream_t stream) {
   if (q4_rows_shape(wq.n + wk.n + wv.n, wk.n < wq.n ? wk.n : wq.n, n_blocks, batch, false, scratch))
     return launch_q4_rows_qkv(s, x, wq, wk, wv, n_blocks, q_out, k_cache, v_cache, pos, batch,
-                              status, scratch, stream);
+                              scratch, stream);
   switch (q4_split(n_blocks)) {
     case 1: return launch_qkv_split<1>(s, x, wq, wk, wv, n_blocks, q_out, k_cache, v_cache, pos, batch, status, stream);
     case 2: return launch_qkv_split<2>(s, x, wq, wk, wv, n_blocks, q_out, k_cache, v_cache, pos, batch, status, stream);

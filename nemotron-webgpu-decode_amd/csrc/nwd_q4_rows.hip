@@ -60,7 +60,7 @@ struct RowsArgs {
   const int32_t* pos;
   int n_kv, head_dim, cap, q16;
   int64_t cache_size;     // elements of one cache
-  int* status;
+  Q4Scratch scratch;      // for the checked build's bounds and its status word
   unsigned long long* records;  // greedy pick
   int per_row;
   unsigned long long* wide_best;  // [rows] picks of wide rows, and the arrivals
@@ -91,6 +91,11 @@ __device__ inline Q4Mat matrix_of(const RowsArgs& p, int& col0) {
     }
   }
   return m;
+}
+
+// The checked build's test of a store of n bytes into the workspace.
+__device__ inline bool in_scratch(const Q4Scratch& s, const void* at, int64_t n) {
+  return in_bounds(static_cast<const char*>(at) - static_cast<const char*>(s.base), n, (int64_t)s.bytes, s.status);
 }
 
 __device__ inline f16x2 twice(uint32_t h) {  // the low half in both
@@ -126,7 +131,9 @@ __device__ inline f16x8 unpack(uint32_t t, uint32_t z) {
 template <int kKind>
 __device__ inline void put(const RowsArgs& p, int row, int col, float v) {
   if constexpr (kKind == kRowsPlain) {
-    float* y = p.y + (int64_t)row * p.cols + col;
+    const int64_t at = (int64_t)row * p.cols + col;
+    if (!in_bounds(at, 1, (int64_t)p.rows * p.cols, p.scratch.status)) return;
+    float* y = p.y + at;
     if (p.epilogue == kQ4Relu2) {
       const float t = fmaxf(v, 0.f);
       v = t * t;
@@ -137,6 +144,7 @@ __device__ inline void put(const RowsArgs& p, int row, int col, float v) {
   } else if constexpr (kKind == kRowsQkv) {
     if (col < p.m[0].n) {
       const int64_t at = (int64_t)row * p.m[0].n + col;
+      if (!in_bounds(at, 1, (int64_t)p.rows * p.m[0].n, p.scratch.status)) return;
       if (p.q16)
         static_cast<f16*>(p.q_out)[at] = (f16)v;
       else
@@ -150,13 +158,23 @@ __device__ inline void put(const RowsArgs& p, int row, int col, float v) {
     if (!is_k) col -= p.m[1].n;
     const int t = p.pos[row];
     if (t < 0 || t >= p.cap) {
-      if (col == 0) atomicOr(p.status, kStatusBadPos);
+      if (col == 0) atomicOr(p.scratch.status, kStatusBadPos);
       return;
     }
     const int64_t at = cache_index_d(row, t, col / p.head_dim, col % p.head_dim, p.n_kv, p.cap, p.head_dim);
-    if (!in_bounds(at, 1, p.cache_size, p.status)) return;
+    if (!in_bounds(at, 1, p.cache_size, p.scratch.status)) return;
     (is_k ? p.k_cache : p.v_cache)[at] = (f16)v;
   }
+}
+
+// A logit of a greedy pick, where they are asked for, and a record.
+__device__ inline void put_logit(const RowsArgs& p, int row, int col, float v) {
+  const int64_t at = (int64_t)row * p.cols + col;
+  if (p.y && in_bounds(at, 1, (int64_t)p.rows * p.cols, p.scratch.status)) p.y[at] = v;
+}
+__device__ inline void put_record(const RowsArgs& p, int row, int i, unsigned long long v) {
+  unsigned long long* at = p.records + (int64_t)row * p.per_row + i;
+  if (in_scratch(p.scratch, at, 8)) *at = v;
 }
 
 // ------------------------------------------------------------ activation rows
@@ -180,7 +198,8 @@ __global__ __launch_bounds__(kRowsThreads) void q4_rows_kernel(const float* __re
                                                                u32x4* __restrict__ a,
                                                                float* __restrict__ factor,
                                                                unsigned long long* __restrict__ wide_best,
-                                                               int* __restrict__ wide_tickets) {
+                                                               int* __restrict__ wide_tickets,
+                                                               const Q4Scratch scratch) {
   __shared__ uint32_t wave_max[kRowsThreads / 64], wave_low[kRowsThreads / 64];
   const int row = blockIdx.x, t = threadIdx.x, runs = n_blocks * 4;
   const f32x4* xr = reinterpret_cast<const f32x4*>(x + (int64_t)row * n_blocks * 32);
@@ -228,10 +247,12 @@ __global__ __launch_bounds__(kRowsThreads) void q4_rows_kernel(const float* __re
   const int e = min(141 - (int)(m >> 23), 126);
   const float up = finite ? __uint_as_float((uint32_t)(e + 127) << 23) : 0.f;
   if (t == 0) {
-    wide_best[row] = 0ull;
-    if (row == 0) *wide_tickets = 0;
-    factor[row] = !finite ? __uint_as_float(0x7FC00000u)
-                          : (wide ? kWideRow : __uint_as_float((uint32_t)(127 - e) << 23));
+    if (in_bounds(row, 1, reinterpret_cast<unsigned long long*>(wide_tickets) - wide_best, scratch.status))
+      wide_best[row] = 0ull;
+    if (row == 0 && in_scratch(scratch, wide_tickets, 4)) *wide_tickets = 0;
+    if (in_bounds(row, 1, reinterpret_cast<float*>(wide_best) - factor, scratch.status))
+      factor[row] = !finite ? __uint_as_float(0x7FC00000u)
+                            : (wide ? kWideRow : __uint_as_float((uint32_t)(127 - e) << 23));
   }
 #pragma unroll
   for (int j = 0; j < kRowsRuns; ++j) {
@@ -248,11 +269,13 @@ __global__ __launch_bounds__(kRowsThreads) void q4_rows_kernel(const float* __re
     const int blk = i >> 2, g = i & 3;
     if (packed) {
       u32x4* o = a + (int64_t)blk * 64 + g * 16 + row;
+      if (!in_bounds(o - a, 9, reinterpret_cast<u32x4*>(factor) - a, scratch.status)) continue;
       o[0] = __builtin_bit_cast(u32x4, hi);
       o[8] = __builtin_bit_cast(u32x4, lo);
     } else {
       const int64_t at = (int64_t)(row >> 4) * n_blocks + blk;
       u32x4* o = a + at * 128 + g * 16 + (row & 15);
+      if (!in_bounds(o - a, 65, reinterpret_cast<u32x4*>(factor) - a, scratch.status)) continue;
       o[0] = __builtin_bit_cast(u32x4, hi);
       o[64] = __builtin_bit_cast(u32x4, lo);
     }
@@ -508,14 +531,14 @@ __global__ __launch_bounds__(kWaves * 64, kTiles == 4 ? 2 : 4) void q4_product_k
         }
         v *= sum_factor(__shfl(factors, mt * kRows + (r < kRows ? r : 0), 64));
         if constexpr (kKind == kRowsArgmax) {  // one record per row and workgroup
-          if (live && p.y) p.y[(int64_t)row * p.cols + cl] = v;
+          if (live) put_logit(p, row, cl, v);
           unsigned long long best = live ? argmax_enc(v, cl, argmax_shape(p.cols)) : 0ull;
 #pragma unroll
           for (int m = kWgCols / 2; m >= 1; m >>= 1) {
             const unsigned long long o = __shfl_xor(best, m, 64);
             best = o > best ? o : best;
           }
-          if (cc == 0 && r < kRows && row < p.rows) p.records[(int64_t)row * p.per_row + blockIdx.x] = best;
+          if (cc == 0 && r < kRows && row < p.rows) put_record(p, row, blockIdx.x, best);
         } else {
           if (live) put<kKind>(p, row, cl, v);
         }
@@ -704,7 +727,7 @@ __global__ __launch_bounds__(kPickThreads) __attribute__((amdgpu_waves_per_eu(2,
       }
       v *= factor;
       if (live_row && cl < p.cols) {
-        if (p.y) p.y[(int64_t)row * p.cols + cl] = v;
+        put_logit(p, row, cl, v);
         const unsigned long long e = argmax_enc(v, cl, shape);
         best = e > best ? e : best;
       }
@@ -716,7 +739,7 @@ __global__ __launch_bounds__(kPickThreads) __attribute__((amdgpu_waves_per_eu(2,
     const unsigned long long o = __shfl_xor(best, i, 64);
     best = o > best ? o : best;
   }
-  if (cc == 0 && live_row) p.records[(int64_t)row * p.per_row + slot] = best;
+  if (cc == 0 && live_row) put_record(p, row, slot, best);
 }
 
 // The picks of q4_pick_kernel's records, a workgroup per row; and the wide
@@ -742,7 +765,8 @@ __global__ __launch_bounds__(kPickMergeThreads) void q4_pick_merge_kernel(const 
   if ((int)blockIdx.x < p.rows && !((wide >> blockIdx.x) & 1)) {
     if (tid == 0) best = 0ull;
     __syncthreads();
-    const unsigned long long e = wave_max_u64(tid < p.per_row ? p.records[(int64_t)blockIdx.x * p.per_row + tid] : 0ull);
+    const unsigned long long* rec = p.records + (int64_t)blockIdx.x * p.per_row + tid;
+    const unsigned long long e = wave_max_u64(tid < p.per_row && in_scratch(p.scratch, rec, 8) ? *rec : 0ull);
     if ((tid & 63) == 0) atomicMax(&best, e);
     __syncthreads();
     if (tid == 0) out[blockIdx.x] = argmax_decode(best, shape);
@@ -781,14 +805,15 @@ __global__ __launch_bounds__(kPickMergeThreads) void q4_pick_merge_kernel(const 
       v = sum8(v);
       v += dpp_mov<kDppRowMirror>(v);
       if (part == 0) {
-        if (p.y) p.y[(int64_t)row * p.cols + col] = v;
+        put_logit(p, row, col, v);
         const unsigned long long c = argmax_enc(v, col, shape);
         e = c > e ? c : e;
       }
     }
     if (e) atomicMax(&best, e);
     __syncthreads();
-    if (tid == 0) __hip_atomic_fetch_max(p.wide_best + row, best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0 && in_scratch(p.scratch, p.wide_best + row, 8))
+      __hip_atomic_fetch_max(p.wide_best + row, best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   if (tid == 0)
     last = __hip_atomic_fetch_add(p.wide_tickets, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
@@ -896,8 +921,10 @@ int rows_per_launch(int cols, int n_blocks, int rows, bool pick, size_t scratch)
 template <int kKind>
 hipError_t launch_rows(RowsArgs p, const float* x, Q4Scratch scratch, uint32_t* out, hipStream_t stream) {
   const int rows = p.rows, nb = p.n_blocks;
-  p.x = x;
   const RowsLayout at = rows_layout(p.cols, nb, rows, kKind == kRowsArgmax);
+  p.x = x;
+  p.scratch = scratch;
+  p.scratch.bytes = at.bytes;
   char* base = static_cast<char*>(scratch.base);
   p.a = reinterpret_cast<const u32x4*>(base);
   float* factor = reinterpret_cast<float*>(base + at.factor);
@@ -911,7 +938,7 @@ hipError_t launch_rows(RowsArgs p, const float* x, Q4Scratch scratch, uint32_t* 
       const bool packed = rows <= kPackedRows;
       const int tiles = pick_tiles(rows);
       q4_rows_kernel<<<rows, kRowsThreads, 0, stream>>>(x, nb, packed ? 1 : 0, reinterpret_cast<u32x4*>(base), factor,
-                                                        p.wide_best, p.wide_tickets);
+                                                        p.wide_best, p.wide_tickets, p.scratch);
       hipError_t e = hipGetLastError();
       const void* kern = packed ? reinterpret_cast<const void*>(q4_pick_kernel<0>)
                                 : reinterpret_cast<const void*>(q4_pick_kernel<1>);
@@ -929,7 +956,7 @@ hipError_t launch_rows(RowsArgs p, const float* x, Q4Scratch scratch, uint32_t* 
   }
   const RowsPlan plan = rows_plan(p.cols, nb, rows);
   q4_rows_kernel<<<rows, kRowsThreads, 0, stream>>>(x, nb, plan.tiles == 0 ? 1 : 0, reinterpret_cast<u32x4*>(base),
-                                                    factor, p.wide_best, p.wide_tickets);
+                                                    factor, p.wide_best, p.wide_tickets, p.scratch);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const int wg_cols = plan.cols * 16, wg_rows = plan.tiles ? 16 * plan.tiles : kPackedRows;
@@ -991,8 +1018,7 @@ hipError_t launch_q4_rows_gemv(const float* x, const Q4Mat& w, int n_blocks, flo
 
 hipError_t launch_q4_rows_qkv(const Shape& s, const float* x, const Q4Mat& wq, const Q4Mat& wk,
                               const Q4Mat& wv, int n_blocks, void* q_out, void* k_cache,
-                              void* v_cache, const int32_t* pos, int batch, int* status,
-                              Q4Scratch scratch, hipStream_t stream) {
+                              void* v_cache, const int32_t* pos, int batch, Q4Scratch scratch, hipStream_t stream) {
   const Q4Mat m[3] = {wq, wk, wv};
   const int per = rows_per_launch(wq.n + wk.n + wv.n, n_blocks, batch, false, scratch.bytes);
   const int64_t seq = (int64_t)s.n_kv * s.cap * s.head_dim;  // cache elements per sequence
@@ -1008,7 +1034,6 @@ hipError_t launch_q4_rows_qkv(const Shape& s, const float* x, const Q4Mat& wq, c
     p.cap = s.cap;
     p.q16 = s.q16;
     p.cache_size = p.rows * seq;
-    p.status = status;
     const hipError_t e = launch_rows<kRowsQkv>(p, x + (int64_t)r * n_blocks * 32, scratch, nullptr, stream);
     if (e != hipSuccess) return e;
   }

@@ -190,6 +190,57 @@ def test_q4_checked_build_matches():
         _same(lambda c, i: c.argmax(logits, 50000, i, B), prod, chk, [ids])
 
 
+@pytest.mark.parametrize("n,nb,rows,heads,cap", [
+    (8192, 98, 3, 32, 64),      # packed
+    (1007, 98, 16, 32, 64), (1007, 98, 30, 32, 64), (3136, 160, 64, 32, 64),
+    (5120, 98, 300, 32, 64),    # four wavefronts
+    (1024, 256, 150, 4, 16),    # several launches, the workspace full
+])
+def test_q4_rows_checked_build_matches(n, nb, rows, heads, cap):
+    """Projections of several rows on the matrix cores, a wide row among
+    them: nothing flagged, the product build's bits."""
+    say("check build q4 rows", n, nb, rows)
+    g = rng(12)
+    prod, chk = _pair(heads, heads, cap, q_dtype="f32", o_dtype="f32", kv_dtype="f32")
+    with prod, chk:
+        x = g.standard_normal((rows, nb * 32)).astype(np.float32)
+        x[1, 40] = 1e9
+        t, w = _q4(g, n, nb)
+        y = torch.zeros((rows, n), dtype=torch.float32, device="cuda")
+        _same(lambda c, o: c.q4_gemv(dev(x), w, o, rows), prod, chk, [y])
+
+
+@pytest.mark.parametrize("n,nb,rows", [(20011, 98, 5), (20011, 98, 40), (20480, 105, 20), (16400, 20, 100)])
+def test_lm_head_rows_checked_build_matches(n, nb, rows):
+    """The wide pick, packed and of three row tiles, and the other kernel's
+    records."""
+    say("check build lm_head rows", n, nb, rows)
+    g = rng(13)
+    prod, chk = _pair(8, 8, 64, q_dtype="f32", o_dtype="f32", kv_dtype="f32")
+    with prod, chk:
+        x = g.standard_normal((rows, nb * 32)).astype(np.float32)
+        x[1, 40] = 1e9
+        t, w = _q4(g, n, nb)
+        logits = torch.zeros((rows, n), dtype=torch.float32, device="cuda")
+        ids = torch.zeros((rows,), dtype=torch.int32, device="cuda")
+        _same(lambda c, lg, i: c.lm_head_argmax(dev(x), w, i, logits=lg, batch=rows), prod, chk,
+              [logits, ids])
+
+
+def test_qkv_rows_checked_build_matches():
+    say("check build qkv rows")
+    g = rng(14)
+    B, H, Hkv, cap, nb = 9, 32, 8, 64, 98
+    prod, chk = _pair(H, Hkv, cap, max_batch=B, q_dtype="f16", o_dtype="f32", kv_dtype="f32")
+    with prod, chk:
+        x = g.standard_normal((B, nb * 32)).astype(np.float32)
+        x[1, 40] = 1e9
+        (tq, wq), (tk, wk), (tv, wv) = _q4(g, H * D, nb), _q4(g, Hkv * D, nb), _q4(g, Hkv * D, nb)
+        qo = torch.zeros((B, H * D), dtype=torch.float16, device="cuda")
+        kc = torch.zeros((B, Hkv, cap, D), dtype=torch.float16, device="cuda")
+        pos = pos_tensor([b * 7 for b in range(B - 1)] + [cap - 1])
+        _same(lambda c, o, k, v: c.qkv_append(dev(x), wq, wk, wv, o, k, v, pos, B), prod, chk,
+              [qo, kc, kc.clone()])
 
 @pytest.mark.parametrize("Dh,H,Hkv", [(96, 6, 2), (100, 3, 3), (300, 2, 1), (128, 7, 1), (128, 12, 4),
                                       (64, 8, 2), (256, 10, 2), (128, 32, 2), (96, 18, 2),
