@@ -36,6 +36,8 @@
 #include "nwd_common.h"
 #include "nwd_internal.h"
 
+#include <atomic>
+
 namespace nwd {
 
 namespace {
@@ -918,6 +920,22 @@ int rows_per_launch(int cols, int n_blocks, int rows, bool pick, size_t scratch)
   return 0;
 }
 
+// The dynamic LDS exceeds the 64 KB default: raises the kernel's limit once
+// per device (the attribute is per device).
+template <auto kKernel>
+hipError_t raise_lds_limit() {
+  static std::atomic<uint64_t> attr_set{0};
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  const uint64_t bit = 1ull << (dev & 63);
+  if (attr_set.load() & bit) return hipSuccess;
+  e = hipFuncSetAttribute(reinterpret_cast<const void*>(kKernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                          160 * 1024);
+  if (e == hipSuccess) attr_set.fetch_or(bit);
+  return e;
+}
+
 template <int kKind>
 hipError_t launch_rows(RowsArgs p, const float* x, Q4Scratch scratch, uint32_t* out, hipStream_t stream) {
   const int rows = p.rows, nb = p.n_blocks;
@@ -940,10 +958,7 @@ hipError_t launch_rows(RowsArgs p, const float* x, Q4Scratch scratch, uint32_t* 
       q4_rows_kernel<<<rows, kRowsThreads, 0, stream>>>(x, nb, packed ? 1 : 0, reinterpret_cast<u32x4*>(base), factor,
                                                         p.wide_best, p.wide_tickets, p.scratch);
       hipError_t e = hipGetLastError();
-      const void* kern = packed ? reinterpret_cast<const void*>(q4_pick_kernel<0>)
-                                : reinterpret_cast<const void*>(q4_pick_kernel<1>);
-      if (e == hipSuccess)
-        e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+      if (e == hipSuccess) e = packed ? raise_lds_limit<q4_pick_kernel<0>>() : raise_lds_limit<q4_pick_kernel<1>>();
       if (e != hipSuccess) return e;
       if (packed)
         q4_pick_kernel<0><<<tiles * p.per_row, kPickThreads, pick_lds(nb), stream>>>(p, tiles);
@@ -968,9 +983,7 @@ hipError_t launch_rows(RowsArgs p, const float* x, Q4Scratch scratch, uint32_t* 
   const int lds = split == groups ? (weights > sums ? weights : sums) : weights + sums;
 #define NWD_ROWS_CASE(T, C, W)                                                                \
   if (plan.tiles == T && plan.cols == C && plan.waves == W) {                                 \
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(q4_product_kernel<T, C, W, kKind>), \
-                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);          \
-    if (e != hipSuccess) return e;                                                            \
+    if ((e = raise_lds_limit<q4_product_kernel<T, C, W, kKind>>()) != hipSuccess) return e;   \
     q4_product_kernel<T, C, W, kKind><<<grid, W * 64, lds, stream>>>(p);                      \
     if ((e = hipGetLastError()) != hipSuccess || kKind != kRowsArgmax) return e;              \
     return launch_argmax_merge(p.records, p.per_row, p.cols, out, rows, stream);              \

@@ -1,6 +1,8 @@
-"""Source check of the bounds-checked build: the kernels of
-csrc/nwd_q4_rows.hip compare every store into an output, a cache or the
-workspace with its buffer (in_bounds, or in_scratch for the workspace).
+"""Source checks of the launchers and of the bounds-checked build.
+
+In the bounds-checked build the kernels of csrc/nwd_q4_rows.hip compare every
+store into an output, a cache or the workspace with its buffer (in_bounds, or
+in_scratch for the workspace).
 
 Every statement of its device code that stores through one of those pointers
 must hold such a check, or follow one that leaves (return, continue) directly
@@ -47,3 +49,18 @@ def test_every_store_is_checked():
     bad, seen = _unchecked(SRC.read_text())
     assert seen >= 11, f"only {seen} stores found"
     assert not bad, bad
+
+
+def test_lds_limits_are_raised_once_per_device():
+    """hipFuncSetAttribute (a runtime call of its own, which a call of few
+    microseconds shows) is not part of every launch: a per-device bit goes
+    before it in its function."""
+    seen = 0
+    for path in sorted(SRC.parent.glob("*")):
+        if path.suffix not in (".h", ".hip"):
+            continue
+        for block in re.split(r"\n}", path.read_text()):  # top-level functions
+            for m in re.finditer(r"hipFuncSetAttribute\(", block):
+                seen += 1
+                assert "attr_set.load()" in block[:m.start()], path.name
+    assert seen >= 4
