@@ -176,14 +176,15 @@ struct Q4Scratch {
 
 // Whether the matrix-core kernels take a projection of n columns (all three
 // for q/k/v, `narrowest` the fewest of them) and `rows` rows; pick: with the
-// greedy pick. Below the products of rows and 32-weight cells here the
-// one-row kernels are faster, whose one launch and 2-5 us per million cells
-// and row stand against two launches (us per call, one-row against matrix-
-// core, K and columns as given: 3136 x 7168, 2 and 3 rows 10.5 against 11.0
-// and 14.8 against 11.2; 5120 x 3136, 2 and 3 rows 9.0 against 10.1 and 11.8
-// against 10.3; 3136 x 1024, 8 rows 6.6 against 8.3; 896 x 896, 32 and 100
-// rows 8.0 against 7.8 and 20.4 against 9.9; with the pick, 1024 x 40000, 4
-// rows 22.9 against 24.3, 3136 x 131072, 2 rows 94 against 87). The others
+// greedy pick. From the products of rows and 32-weight cells here on (below,
+// the one-row kernels' one launch stands against two) they do where an
+// estimate of both (nwd_q4_rows.hip) has them faster. us per call, one-row
+// against matrix-core, K and columns as given: 3136 x 7168, 2 and 3 rows 10.5
+// against 11.0 and 14.8 against 11.2; 5120 x 3136, 2 and 3 rows 9.0 against
+// 10.1 and 11.8 against 10.3; 3136 x 1024, 8 rows 6.8 against 8.2; 896 x 896,
+// 32 and 100 rows 8.0 against 7.8 and 20.4 against 9.9; with the pick, 3136 x
+// 131072, 2 rows 87 against 77, x 32768 27.6 against 27.8, 2048 x 32768, 2 and
+// 3 rows 19.8 against 22.4 and 25.3 against 22.9. The other bounds
 // are what their reads need: 16 cells (one 8-byte run of zero points), byte
 // offsets below 2^31, and scratch for at least 8 rows.
 bool q4_rows_shape(int n, int narrowest, int n_blocks, int rows, bool pick, Q4Scratch scratch);

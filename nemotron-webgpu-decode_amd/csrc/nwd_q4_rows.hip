@@ -1006,13 +1006,51 @@ RowsArgs rows_args(const Q4Mat* m, int n_mats, int n_blocks) {
   return p;
 }
 
+// Estimates of a call on either kind of kernel, us, of which the less decides
+// (q4_rows_shape). The one-row kernels stream their columns' weights once per
+// row, at any size; a workgroup here takes a row group through all of K,
+// however few workgroups there are, so that few columns with a long K leave
+// most of the chip idle for that long. One-row against matrix-core, us: K =
+// 8192, 64 columns, 96 rows 9.5 against 31.6, 512 columns, 17 rows 13.5
+// against 18.8, 2048 columns, 3 rows 11.3 against 12.5; K = 3136, 256
+// columns, 64 rows 10.3 against 16.6; K = 5120, 100 columns, 96 rows 12.0
+// against 24.2; with the pick, K = 4096, 131072 columns, 2 rows 121 against
+// 149 and K = 896 31 against 43. Over K of 32 to 8192, 16 to 16384 columns (picks
+// 4096 to 131072) and 2 to 128 rows the estimates lie within 20% of nearly all
+// times, the choice within 4% of the better kind wherever it takes this one,
+// and loses at most 15% where it leaves it.
+double one_row_us(int cols, int n_blocks, int rows, bool pick) {
+  const double nb = n_blocks, merge = pick ? 3 : 0;
+  // lm_head's form (128-thread workgroups, K in registers), per column and row
+  if (pick && cols >= 16384) return 5 + merge + 1e-3 * rows * cols * (0.03 + (0.0019 + 0.000011 * nb) * nb);
+  return 3 + merge + 1e-3 * rows * ((cols + 15) / 16) * (0.8 + 0.07 * nb);
+}
+double several_rows_us(int cols, int n_blocks, int rows, bool pick) {
+  const double nb = n_blocks, merge = pick ? 3 : 0;
+  if (pick && pick_wide(cols, n_blocks, rows))
+    return 8.5 + merge + 1e-3 * pick_tiles(rows) * cols * (0.15 + 0.0036 * nb);
+  const RowsPlan p = rows_plan(cols, n_blocks, rows);
+  // a row group's time per block of K, by row tiles (packed, 1, 2, 4) and column tiles
+  constexpr double kGroup[2][4] = {{0.019, 0.025, 0.046, 0.100}, {0.059, 0.073, 0.109, 0.124}};
+  const int wg_rows = p.tiles ? 16 * p.tiles : kPackedRows, groups = (rows + wg_rows - 1) / wg_rows;
+  const int64_t wgs = (cols + 16 * p.cols - 1) / (16 * p.cols) * (int64_t)p.split;
+  const int64_t slots = p.waves == 4 ? 512 : 256, rounds = (wgs + slots - 1) / slots;
+  return 7 + merge + kGroup[p.cols - 1][p.tiles == 4 ? 3 : p.tiles] * nb * rounds *
+                         ((groups + p.split - 1) / p.split) * (p.waves == 4 ? 2 : 1);
+}
+
 }  // namespace
 
 bool q4_rows_shape(int n, int narrowest, int n_blocks, int rows, bool pick, Q4Scratch scratch) {
   const int64_t cells = (int64_t)n * n_blocks;
-  return rows >= 2 && cells * rows >= (pick && n >= 16384 ? 6000000 : 1500000) &&
-         (int64_t)narrowest * n_blocks >= 16 && cells * 16 < ((int64_t)1 << 31) - (1 << 20) &&
-         rows_per_launch(n, n_blocks, rows, pick, scratch.bytes) > 0;
+  if (rows < 2 || cells * rows < (pick && n >= 16384 ? 6000000 : 1500000)) return false;
+  if ((int64_t)narrowest * n_blocks < 16 || cells * 16 >= ((int64_t)1 << 31) - (1 << 20)) return false;
+  const int per = rows_per_launch(n, n_blocks, rows, pick, scratch.bytes);
+  if (per == 0) return false;
+  const int rest = rows % per;
+  double several = rows / per * several_rows_us(n, n_blocks, per, pick);
+  if (rest) several += several_rows_us(n, n_blocks, rest, pick);
+  return several < one_row_us(n, n_blocks, rows, pick);
 }
 
 hipError_t launch_q4_rows_gemv(const float* x, const Q4Mat& w, int n_blocks, float* y, int rows,

@@ -10,8 +10,7 @@ fp16 ulp; the picked token is the largest logit.
 Sizes: the smallest and largest row counts of each row tiling (packed up to
 8, then 16, 32 and 64 rows, several groups of 64), column counts that leave a
 remainder of the 16- and 32-column tiles, odd block counts, one block, and
-the largest K. Each product of rows and cells is past the 1.5 million from
-which these kernels run.
+the largest K. All are sizes that these kernels take (test_route).
 """
 import numpy as np
 import pytest
@@ -57,15 +56,15 @@ def _ctx(H=32, Hkv=8, cap=512, B=64, q="f32", Dh=D):
     (1953, 98, 8),     # packed, full; one column past a tile
     (2050, 97, 9),     # one tile of 16, odd block count
     (1000, 98, 16),
-    (1007, 98, 17),    # two tiles
-    (520, 98, 32),
+    (1607, 98, 17),    # two tiles
+    (1032, 98, 32),
     (3136, 160, 33),   # four tiles, mostly padding; K = 5120
     (7168, 98, 64),    # two column tiles per workgroup
-    (300, 98, 65),     # a second group of one row
+    (904, 98, 65),     # a second group of one row
     (5120, 98, 300),   # four wavefronts per workgroup
     (3136, 160, 200),  # a workgroup walks several groups
-    (37, 130, 320),    # few columns
-    (64, 256, 130),    # the largest K
+    (37, 130, 900),    # few columns
+    (64, 256, 600),    # the largest K
     (48, 1, 40000),    # one block: most wavefronts have none
     (777, 5, 500),
 ])
@@ -87,6 +86,38 @@ def test_rows_match_float64(n, n_blocks, rows):
     t = np.maximum(got, np.float32(0))
     np.testing.assert_array_equal(host(relu), t * t)
     np.testing.assert_array_equal(host(acc), prev + got)
+
+
+def _one_row(ctx, w, x, n):
+    """Every row by itself, on the one-row kernels."""
+    y = torch.empty((len(x), n), dtype=torch.float32, device="cuda")
+    dx = dev(x)
+    for b in range(len(x)):
+        ctx.q4_gemv(dx[b:b + 1], w.w, y[b:b + 1], 1)
+    return host(y)
+
+
+@pytest.mark.parametrize("n,n_blocks,rows,several", [
+    # long K, few columns: faster on the one-row kernels
+    (64, 256, 96, False), (100, 256, 70, False), (256, 98, 64, False), (512, 256, 17, False),
+    (100, 160, 96, False), (2048, 256, 3, False), (5120, 256, 2, False),
+    # and the others
+    (1953, 98, 8, True), (1607, 98, 17, True), (904, 98, 65, True), (37, 130, 900, True),
+    (64, 256, 600, True), (2048, 256, 4, True), (3136, 160, 3, True),
+])
+def test_route(n, n_blocks, rows, several):
+    """The kind of kernel that a call takes, told by its bits: the one-row
+    kernels give a row the same at every batch, those of several rows sum in
+    another order."""
+    say(f"q4 rows route n={n} n_blocks={n_blocks} rows={rows}")
+    g = rng(990)
+    w = Q4(g, n, n_blocks)
+    x = g.standard_normal((rows, 32 * n_blocks)).astype(np.float32)
+    y = torch.empty((rows, n), dtype=torch.float32, device="cuda")
+    with _ctx() as ctx:
+        ctx.q4_gemv(dev(x), w.w, y, rows)
+        same = np.array_equal(host(y), _one_row(ctx, w, x, n))
+    assert same == (not several)
 
 
 def test_rows_in_small_workspace():
@@ -172,7 +203,6 @@ def test_wide_rows(n, n_blocks, rows, head):
         x[b, 32 * blk + b % 32] = large[b // 2 % len(large)]
     x[1, :32] *= np.float32(1e-6)  # the other way about: a block far below the rest
     y = torch.full((rows, n), float("nan"), dtype=torch.float32, device="cuda")
-    one = torch.empty_like(y)
     token = torch.full((rows,), -1, dtype=torch.int32, device="cuda")
     dx = dev(x)
     with _ctx() as ctx:
@@ -180,9 +210,7 @@ def test_wide_rows(n, n_blocks, rows, head):
             ctx.lm_head_argmax(dx, w.w, token, y, rows)
         else:
             ctx.q4_gemv(dx, w.w, y, rows)
-        for b in range(rows):
-            ctx.q4_gemv(dx[b:b + 1], w.w, one[b:b + 1], 1)
-        got, one = host(y), host(one)
+        got, one = host(y), _one_row(ctx, w, x, n)
     y64, bound = w.f64(x)  # the large elements are not in the bound
     assert np.all(np.abs(got - y64) <= TOL_REL * bound)
 
