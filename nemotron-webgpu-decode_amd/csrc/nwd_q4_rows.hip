@@ -1014,29 +1014,34 @@ RowsArgs rows_args(const Q4Mat* m, int n_mats, int n_blocks) {
 // 8192, 64 columns, 96 rows 9.5 against 31.6, 512 columns, 17 rows 13.5
 // against 18.8, 2048 columns, 3 rows 11.3 against 12.5; K = 3136, 256
 // columns, 64 rows 10.3 against 16.6; K = 5120, 100 columns, 96 rows 12.0
-// against 24.2; with the pick, K = 4096, 131072 columns, 2 rows 121 against
-// 149 and K = 896 31 against 43. Over K of 32 to 8192, 16 to 16384 columns (picks
-// 4096 to 131072) and 2 to 128 rows the estimates lie within 20% of nearly all
-// times, the choice within 4% of the better kind wherever it takes this one,
-// and loses at most 15% where it leaves it.
+// against 24.2, 16 columns, 4000 rows 60 against 129; with the pick, K = 4096,
+// 131072 columns, 2 rows 121 against 149 and K = 896 31 against 43. Over K of 32
+// to 8192, 16 to 16384 columns and 2 to 4000 rows (picks: 4096 to 131072 columns, 2 to 64 rows),
+// 2000 shapes past the bound of q4_rows_shape, the choice lost more than 6%
+// against the one-row kernels at one (12%: K = 8192, 48 columns, 2000 rows)
+// and more than 13% against the matrix cores at one (18%: K = 8192, 100
+// columns, 256 rows).
 double one_row_us(int cols, int n_blocks, int rows, bool pick) {
-  const double nb = n_blocks, merge = pick ? 3 : 0;
+  const double nb = n_blocks;
   // lm_head's form (128-thread workgroups, K in registers), per column and row
-  if (pick && cols >= 16384) return 5 + merge + 1e-3 * rows * cols * (0.03 + (0.0019 + 0.000011 * nb) * nb);
-  return 3 + merge + 1e-3 * rows * ((cols + 15) / 16) * (0.8 + 0.07 * nb);
+  if (pick && cols >= 16384) return 8 + 1e-3 * rows * cols * (0.03 + (0.0016 + 0.0000125 * nb) * nb);
+  // per 16 columns and row, by the wavefronts that share K (q4_split)
+  const double unit = nb < 64 ? 1.8 + 0.038 * nb : (nb < 128 ? 2.6 + 0.0475 * nb : 4.8 + 0.052 * nb);
+  return (pick ? 8 : 3) + 1e-3 * rows * ((cols + 15) / 16) * unit;
 }
 double several_rows_us(int cols, int n_blocks, int rows, bool pick) {
-  const double nb = n_blocks, merge = pick ? 3 : 0;
-  if (pick && pick_wide(cols, n_blocks, rows))
-    return 8.5 + merge + 1e-3 * pick_tiles(rows) * cols * (0.15 + 0.0036 * nb);
+  const double nb = n_blocks;
+  if (pick && pick_wide(cols, n_blocks, rows)) return 11.5 + 1e-3 * pick_tiles(rows) * cols * (0.15 + 0.0036 * nb);
   const RowsPlan p = rows_plan(cols, n_blocks, rows);
   // a row group's time per block of K, by row tiles (packed, 1, 2, 4) and column tiles
-  constexpr double kGroup[2][4] = {{0.019, 0.025, 0.046, 0.100}, {0.059, 0.073, 0.109, 0.124}};
+  constexpr double kGroup[2][4] = {{0.019, 0.025, 0.046, 0.092}, {0.059, 0.073, 0.109, 0.124}};
   const int wg_rows = p.tiles ? 16 * p.tiles : kPackedRows, groups = (rows + wg_rows - 1) / wg_rows;
   const int64_t wgs = (cols + 16 * p.cols - 1) / (16 * p.cols) * (int64_t)p.split;
   const int64_t slots = p.waves == 4 ? 512 : 256, rounds = (wgs + slots - 1) / slots;
-  return 7 + merge + kGroup[p.cols - 1][p.tiles == 4 ? 3 : p.tiles] * nb * rounds *
-                         ((groups + p.split - 1) / p.split) * (p.waves == 4 ? 2 : 1);
+  const double operands = 1e-3 * rows * nb;  // written and read once, past L2 where many
+  return (pick ? 10 : 7) + (0.1 + 0.0001 * operands) * operands +
+         kGroup[p.cols - 1][p.tiles == 4 ? 3 : p.tiles] * nb * rounds * ((groups + p.split - 1) / p.split) *
+             (p.waves == 4 ? 2 : 1);
 }
 
 }  // namespace

@@ -210,7 +210,7 @@ def test_q4_rows_checked_build_matches(n, nb, rows, heads, cap):
         _same(lambda c, o: c.q4_gemv(dev(x), w, o, rows), prod, chk, [y])
 
 
-@pytest.mark.parametrize("n,nb,rows", [(20011, 98, 5), (20011, 98, 40), (20480, 105, 20), (16400, 20, 100)])
+@pytest.mark.parametrize("n,nb,rows", [(20011, 98, 5), (33001, 98, 40), (20480, 105, 20), (16400, 20, 100)])
 def test_lm_head_rows_checked_build_matches(n, nb, rows):
     """The wide pick, packed and of three row tiles, and the other kernel's
     records."""

@@ -63,8 +63,8 @@ def _ctx(H=32, Hkv=8, cap=512, B=64, q="f32", Dh=D):
     (904, 98, 65),     # a second group of one row
     (5120, 98, 300),   # four wavefronts per workgroup
     (3136, 160, 200),  # a workgroup walks several groups
-    (37, 130, 900),    # few columns
-    (64, 256, 600),    # the largest K
+    (37, 130, 1200),   # few columns
+    (520, 256, 130),   # the largest K
     (48, 1, 40000),    # one block: most wavefronts have none
     (777, 5, 500),
 ])
@@ -102,8 +102,8 @@ def _one_row(ctx, w, x, n):
     (64, 256, 96, False), (100, 256, 70, False), (256, 98, 64, False), (512, 256, 17, False),
     (100, 160, 96, False), (2048, 256, 3, False), (5120, 256, 2, False),
     # and the others
-    (1953, 98, 8, True), (1607, 98, 17, True), (904, 98, 65, True), (37, 130, 900, True),
-    (64, 256, 600, True), (2048, 256, 4, True), (3136, 160, 3, True),
+    (1953, 98, 8, True), (1607, 98, 17, True), (904, 98, 65, True), (37, 130, 1200, True),
+    (520, 256, 130, True), (2048, 256, 4, True), (3136, 160, 3, True),
 ])
 def test_route(n, n_blocks, rows, several):
     """The kind of kernel that a call takes, told by its bits: the one-row
@@ -184,7 +184,7 @@ def _hide_block(w, n, n_blocks, blk):
     (4096, 98, 8, False),     # packed
     (1007, 98, 16, False), (1007, 97, 32, False),
     (3136, 160, 64, False), (5120, 98, 130, False),
-    (16400, 98, 7, True), (20011, 98, 48, True),  # wide picks
+    (16400, 98, 7, True), (33001, 98, 48, True),  # wide picks
     (16400, 105, 16, True),                       # the other kernel's
 ])
 def test_wide_rows(n, n_blocks, rows, head):
@@ -263,7 +263,8 @@ def test_qkv_rows(H, Hkv, q, Dh, B):
 
 
 @pytest.mark.parametrize("n,n_blocks,rows", [(20011, 98, 4), (20011, 98, 16), (16384, 97, 20), (33000, 33, 70),
-                                                (20017, 104, 48), (17001, 8, 48), (20480, 105, 9)])
+                                                (33001, 104, 48), (20017, 104, 48), (17001, 8, 48),
+                                                (20480, 105, 9)])
 def test_lm_head_rows(n, n_blocks, rows):
     say(f"lm_head rows n={n} n_blocks={n_blocks} rows={rows}")
     g = rng(970 + rows)
