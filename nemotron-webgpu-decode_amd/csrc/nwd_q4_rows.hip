@@ -551,7 +551,7 @@ __global__ __launch_bounds__(kWaves * 64, kTiles == 4 ? 2 : 4) void q4_product_k
 
 // ------------------------------------------------------- wide greedy picks
 
-// lm_head with the pick, up to 48 rows: one persistent workgroup per CU. Its
+// lm_head with the pick (pick_wide says which): one persistent workgroup per CU. Its
 // 8 wavefronts split K and hold their part of one row tile's A operands in
 // registers for the whole launch (read per 32 columns, as above, they were
 // more L2 traffic than the weights); the weights of the next 32 columns, one
@@ -876,11 +876,19 @@ RowsPlan rows_plan(int cols, int n_blocks, int rows) {
 }
 
 // The wide pick: its grid, which picks it takes, and its records per row
-// (one per workgroup of a row tile). The limit of K is its registers'; of
-// rows, 131072 x 3136: 48 rows 203 against 210 us, 64 rows 258 against 222.
+// (one per workgroup of a row tile). The limit of K is its registers'. Each
+// further row tile has it read and unpack the weights again: past 32 rows it
+// wins only near its longest K, where the other kernel's 64-row form has one
+// workgroup per CU, and with many columns. 131072 columns, the other kernel
+// against this, us: K = 3136, 16 rows 125 against 75, 32 rows 197 against 135,
+// 48 rows 203 against 195, 64 rows 211 against 252; K = 3328, 48 rows 241
+// against 202; K = 2560, 32 rows 179 against 119, 48 rows 168 against 170; K =
+// 896, 32 rows 93 against 79, 48 rows 96 against 113; 32768 columns, K = 3136,
+// 48 rows 62 against 63.
 constexpr int kPickGrid = 256;
 bool pick_wide(int cols, int n_blocks, int rows) {
-  return cols >= 16384 && n_blocks <= kPickMaxBlocks && rows <= 48;
+  return cols >= 16384 && n_blocks <= kPickMaxBlocks &&
+         (rows <= 32 || (rows <= 48 && n_blocks > 96 && cols > 32768));
 }
 int pick_tiles(int rows) { return rows <= kPackedRows ? 1 : (rows + 15) / 16; }
 int records_per_row(int cols, int n_blocks, int rows) {

@@ -282,6 +282,24 @@ def test_lm_head_rows(n, n_blocks, rows):
     np.testing.assert_array_equal(tok[1], tok[0])
 
 
+@pytest.mark.parametrize("n,n_blocks,rows,wide", [(33001, 97, 33, True), (20011, 98, 33, False),
+                                                  (33001, 20, 40, False)])
+def test_pick_route(n, n_blocks, rows, wide):
+    """Picks of 33 to 48 rows: on the wide pick kernel, which gives a row of
+    every row tile the bits of its 16-row form, or on the other, whose
+    64-row form sums in another order."""
+    say(f"lm_head route n={n} n_blocks={n_blocks} rows={rows}")
+    g = rng(981)
+    w = Q4(g, n, n_blocks)
+    dx = dev(g.standard_normal((rows, 32 * n_blocks)).astype(np.float32))
+    many, few = (torch.empty((r, n), dtype=torch.float32, device="cuda") for r in (rows, 16))
+    token = torch.empty(rows, dtype=torch.int32, device="cuda")
+    with _ctx() as ctx:
+        ctx.lm_head_argmax(dx, w.w, token, many, rows)
+        ctx.lm_head_argmax(dx[16:32], w.w, token, few, 16)
+        assert np.array_equal(host(many)[16:32], host(few)) == wide
+
+
 def test_lm_head_fills_the_workspace():
     """Batches up to the largest that the workspace takes (128 rows of 1024
     records here, its 1 MiB) run the kernels of several rows as they do in a
