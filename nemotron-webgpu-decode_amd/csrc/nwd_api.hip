@@ -104,8 +104,9 @@ int resolve_len(const nwd_ctx* ctx, int32_t max_len) {
 // with 16 against 60.2 with 17; B = 4 at 32K, 82.4 with 8 against 95.0 with
 // 17. Larger batches fill the chip by themselves and keep the 2048-key
 // bound per split, which evens out ragged lengths (64 sequences of
-// 512-16384 keys run 9 splits each).
-int auto_splits(int n_heads, int n_kv_heads, int batch, int max_len) {
+// 512-16384 keys run 9 splits each); those short of a whole wave have their
+// own counts below.
+int auto_splits(int n_heads, int n_kv_heads, int head_dim, int batch, int max_len) {
   const int units = (max_len + kMinKeysPerSplit - 1) / kMinKeysPerSplit;
   const int64_t heads = (int64_t)batch * n_heads;
   if (heads <= nwd::kSubSplitMaxWorkgroups) {
@@ -138,25 +139,35 @@ int auto_splits(int n_heads, int n_kv_heads, int batch, int max_len) {
   int n = (kTargetWorkgroups + per_wave - 1) / per_wave;              // fill the chip
   const int by_len = (max_len + kMaxKeysPerSplit - 1) / kMaxKeysPerSplit;  // bound per-split work
   // Between half a wave and a whole one, two splits make a second wave that
-  // is nearly empty at the low end, and cost records at every length. Up to
-  // 2048 keys one split wins where a workgroup serves several heads; past
-  // that, and for single heads, splits of about 512 keys, up to 8, even the
-  // waves out where the splits so far leave a quarter of theirs idle. us per
-  // call, this against the two splits (4 at 8000 keys) before, equal lengths
-  // / lengths from an eighth up: 32q/8kv/d128, batch 17, 300 keys 8.2 / 7.6
-  // against 11.4 / 10.8, 1800 24.6 / 23.2 against 31.5 / 26.8, 4000 47.9 /
-  // 35.0 against 64.3 / 50.5, 8000 95.1 / 65.9 against 106.6 / 69.2; batch
-  // 30, 1800 keys 34.9 / 26.3 against 37.5 / 26.5; 16q/8kv/d256, batch 20,
-  // 2500 72.8 / 48.0 against 78.0 / 61.6; 32q/32kv/d96, batch 6, 1500 22.5 /
-  // 18.2 against 23.7 / 19.4; 32q/8kv/d64, batch 22, 2500 22.9 / 20.0 against
-  // 24.7 / 19.5. Where the waves were full it lost: 32q/8kv, batch 27, 2500
-  // keys 47.9 against 47.0, batch 31, 4000 85.7 against 84.2.
+  // is nearly empty at the low end, and cost records at every length. Short
+  // lengths run one split: up to 800 keys with groups of four heads and up
+  // at head sizes to 128, else 400. max_len bounds all lengths, so the counts are chosen over
+  // batches of equal lengths, of lengths from an eighth up, of one long
+  // sequence among short ones and of both by halves: us per call of one split
+  // against two, 32q/8kv/d128, batch 17, 640 keys, the first three of these
+  // 11.8 / 11.0 / 10.8 against 16.0 / 11.9 / 11.6; batch 22, 800 keys 0.78,
+  // 0.89 and 0.99 of two splits' times; but 1000 keys 0.82, 0.92 and 1.07, 2000
+  // keys 0.82, 0.98 and 1.28; 24q/8kv (group 3), batch 17, 400 keys 0.80, 0.89
+  // and 0.89, 700 keys with lengths from an eighth up 13.1 against 11.7;
+  // 10q/2kv/d256, batch 65, 700 keys the same way 23.5 against 20.3. Past 2304 keys
+  // splits of about 512 keys, up to 8, even the waves out where that makes
+  // waves times keys a fifth less: batch 17, 2600 keys 0.82, 0.97 and 0.90 of
+  // two splits' times, batch 19, 3500 keys 0.83, 0.68 and 0.77; at 2100 keys
+  // 1.00 to 1.11 for some batches, and at head size 64, with half the bytes a
+  // key, 1.05 to 1.18 up to 6500 keys. Single heads gain from any length on:
+  // 32q/32kv/d96, batch 5, 1500 keys 0.92 and 0.94.
+  // Over 17 layouts and these lengths the mean is 0.78 of two splits' times,
+  // the worst of 1788 batches 1.05.
   if (per_wave < kTargetWorkgroups) {
-    if (n_heads > n_kv_heads && max_len <= 2048) return 1;
-    const int64_t wgs = (int64_t)per_wave * (by_len > n ? by_len : n);
-    const int64_t waves = (wgs + kTargetWorkgroups - 1) / kTargetWorkgroups;
+    const bool groups = n_heads > n_kv_heads;
+    if (groups && max_len <= (n_heads >= 4 * n_kv_heads && head_dim <= 128 ? 800 : 400)) return 1;
+    const int now = by_len > n ? by_len : n;
     const int by_wave = (max_len + 511) / 512 < 8 ? (max_len + 511) / 512 : 8;
-    if (4 * wgs <= 3 * kTargetWorkgroups * waves && by_wave > n) n = by_wave;
+    const auto waves = [&](int k) { return ((int64_t)per_wave * k + kTargetWorkgroups - 1) / kTargetWorkgroups; };
+    const auto chain = [&](int k) { return waves(k) * ((max_len + k - 1) / k); };  // keys, one after another
+    if (head_dim > 64 && (!groups || max_len > 2304) && by_wave > now &&
+        4 * (int64_t)per_wave * now <= 3 * kTargetWorkgroups * waves(now) && 5 * chain(by_wave) <= 4 * chain(now))
+      n = by_wave;
   }
   if (by_len > n) n = by_len;
   return n < 1 ? 1 : n;
@@ -505,7 +516,7 @@ int32_t nwd_decode_splits(const nwd_ctx* ctx, int32_t batch, int32_t max_len) {
   const nwd::Shape s = route == kRoutePadded ? nwd::padded_shape(ctx->shape) : ctx->shape;
   int n = ctx->forced_splits > 0 ? ctx->forced_splits
           : route == kRouteGeneral ? general_splits(general_units(s, batch, 1), len)
-                                   : auto_splits(s.n_heads, kv_groups(s), batch, len);
+                                   : auto_splits(s.n_heads, kv_groups(s), s.head_dim, batch, len);
   return clamp_splits(ctx, s, batch, n);
 }
 
@@ -605,7 +616,7 @@ int nwd_append_decode_noalloc(const nwd_desc* desc, const void* q, const void* k
   const nwd::Shape sh = shape_of(desc);
   const bool general = decode_route(sh, false) == kRouteGeneral;
   int n = general ? general_splits(general_units(sh, batch, 1), len)
-                  : auto_splits(desc->n_heads, kv_groups(sh), batch, len);
+                  : auto_splits(desc->n_heads, kv_groups(sh), sh.head_dim, batch, len);
   if (n > kMaxSplits) n = kMaxSplits;
   const int64_t records = n > 1 ? (int64_t)batch * desc->n_heads * n : 0;
   const int rw = nwd::record_width(desc->head_dim);  // floats per record

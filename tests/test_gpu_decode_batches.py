@@ -18,14 +18,23 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("H,Hkv,Dh,B,longest,splits", [
-    (32, 8, 128, 17, 2048, 1),  # the longest of one split
-    (32, 8, 128, 17, 2049, 5),
+    (32, 8, 128, 17, 800, 1),   # the longest of one split
+    (32, 8, 128, 17, 801, 2),
+    (32, 8, 128, 17, 2304, 2),
+    (32, 8, 128, 17, 2305, 5),
     (32, 8, 128, 31, 600, 1),
     (32, 8, 128, 30, 2500, 2),  # its two waves are nearly full
     (32, 8, 128, 24, 5000, 8),
-    (32, 32, 96, 6, 1500, 3),   # one head per workgroup
+    (32, 8, 128, 17, 6500, 4),  # waves times keys only a sixth less
+    (24, 8, 128, 17, 400, 1),   # a group below four heads
+    (24, 8, 128, 17, 401, 2),
+    (32, 32, 96, 5, 1500, 3),   # one head per workgroup
+    (32, 32, 96, 6, 1500, 2),   # three waves of a third are two of a half
     (16, 8, 256, 20, 2500, 5),
+    (10, 2, 256, 65, 400, 1),   # head sizes past 128
+    (10, 2, 256, 65, 401, 2),
     (14, 2, 64, 65, 300, 1),
+    (14, 2, 64, 65, 3000, 2),   # not by waves at head size 64
 ])
 def test_batched_step(H, Hkv, Dh, B, longest, splits):
     say(f"batched step H={H} Hkv={Hkv} D={Dh} B={B} longest={longest}")
