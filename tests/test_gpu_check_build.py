@@ -194,7 +194,7 @@ def test_q4_checked_build_matches():
     (8192, 98, 3, 32, 64),      # packed
     (1007, 98, 16, 32, 64), (1007, 98, 30, 32, 64), (3136, 160, 64, 32, 64),
     (5120, 98, 300, 32, 64),    # four wavefronts
-    (1024, 256, 150, 4, 16),    # several launches, the workspace full
+    (2048, 256, 150, 4, 16),    # several launches, the workspace full
 ])
 def test_q4_rows_checked_build_matches(n, nb, rows, heads, cap):
     """Projections of several rows on the matrix cores, a wide row among

@@ -19,6 +19,7 @@ torch = pytest.importorskip("torch")
 
 import nwd_attn as nw  # noqa: E402
 from gpu_util import dev, host, pos_tensor, say  # noqa: E402
+from argmax_cases import reference_rule  # noqa: E402
 from q4_cases import dequant_f64, random_q4, rng  # noqa: E402
 
 pytestmark = pytest.mark.gpu
@@ -67,6 +68,7 @@ def _ctx(H=32, Hkv=8, cap=512, B=64, q="f32", Dh=D):
     (520, 256, 130),   # the largest K
     (48, 1, 40000),    # one block: most wavefronts have none
     (777, 5, 500),
+    (16400, 40, 8), (16400, 40, 16), (16400, 40, 32),  # two column tiles: wide projections
 ])
 def test_rows_match_float64(n, n_blocks, rows):
     say(f"q4 rows n={n} n_blocks={n_blocks} rows={rows}")
@@ -120,21 +122,158 @@ def test_route(n, n_blocks, rows, several):
     assert same == (not several)
 
 
-def test_rows_in_small_workspace():
-    """A context whose workspace holds few activation rows: the call goes
-    through it in several launches."""
-    n, n_blocks, rows = 1024, 256, 150
-    say(f"q4 rows in a small workspace, rows={rows}")
+def _workspace(H, Hkv, cap, B):
+    """Bytes of a context's split-K workspace at head size 128 (nwd_create)."""
+    records = max(H * 256, H // Hkv * 512, B * H, min(2 * cap * H * B, 65536))
+    return records * 512
+
+
+def _launch_rows(n_blocks, rows, workspace, records=lambda rows: 0):
+    """Rows per launch: all, a multiple of 64, 32, 16 or 8, the most whose
+    operands, factors, picks and records the workspace holds (8 rows: high and
+    low parts in one tile of 16 rows, 1 KiB a block; more: 2 KiB a block for
+    each tile of a group of 1, 2 or 4)."""
+    def need(r):
+        tiles = 1 if r <= 16 else 2 if r <= 32 else -(-r // 64) * 4
+        a = n_blocks * (1024 if r <= 8 else 2048 * tiles)
+        return a + -(-r // 4) * 16 + -(-r // 2) * 16 + 16 + 8 * r * records(r)
+
+    sizes = [rows] + list(range((rows - 1) // 64 * 64, 0, -64)) + [32, 16, 8]
+    return next(r for r in sizes if r <= rows and need(r) <= workspace)
+
+
+@pytest.mark.parametrize("heads,per", [(3, 8), (5, 16), (9, 32), (17, 64), (34, 128)])
+def test_rows_in_small_workspace(heads, per):
+    """A context whose workspace holds `per` activation rows: the call goes
+    through it in several launches, the last one ragged, each with the bits
+    that a call of its rows has in a roomy context."""
+    n, n_blocks, rows = 2048, 256, 150
+    say(f"q4 rows in a small workspace, {per} of {rows} rows a launch")
+    assert _launch_rows(n_blocks, rows, _workspace(heads, heads, 16, 1)) == per
     g = rng(950)
     w = Q4(g, n, n_blocks)
     x = g.standard_normal((rows, 32 * n_blocks)).astype(np.float32)
-    for heads in (1, 2, 4):
-        y = torch.full((rows, n), float("nan"), dtype=torch.float32, device="cuda")
-        with _ctx(heads, heads, 16, 1) as ctx:
-            ctx.q4_gemv(dev(x), w.w, y, rows)
-            got = host(y)
-        y64, bound = w.f64(x)
-        assert np.all(np.abs(got - y64) <= TOL_REL * bound), heads
+    dx = dev(x)
+    y = torch.full((rows, n), float("nan"), dtype=torch.float32, device="cuda")
+    parts = torch.empty_like(y)
+    with _ctx(heads, heads, 16, 1) as ctx, _ctx() as roomy:
+        ctx.q4_gemv(dx, w.w, y, rows)
+        for b in range(0, rows, per):
+            m = min(per, rows - b)
+            roomy.q4_gemv(dx[b:b + m], w.w, parts[b:b + m], m)
+        got = host(y)
+        np.testing.assert_array_equal(got, host(parts))
+        assert not np.array_equal(got, _one_row(ctx, w, x, n))
+    y64, bound = w.f64(x)
+    assert np.all(np.abs(got - y64) <= TOL_REL * bound)
+
+
+def test_qkv_rows_in_small_workspace():
+    """The same for q/k/v: queries, caches and positions of every launch, a
+    wide row and a position outside the cache in later ones."""
+    H, Hkv, cap, B, nb = 8, 4, 2, 60, 256
+    say(f"qkv rows in a small workspace, B={B}")
+    per = _launch_rows(nb, B, _workspace(H, Hkv, cap, B))
+    assert per == 16
+    g = rng(955)
+    wq, wk, wv = Q4(g, H * D, nb), Q4(g, Hkv * D, nb), Q4(g, Hkv * D, nb)
+    x = g.standard_normal((B, 32 * nb)).astype(np.float32)
+    x[20, 7] = 1e9
+    pos = [int(v) for v in g.integers(0, cap, size=B)]
+    pos[37] = cap
+    canary = -7.5
+
+    def buffers():
+        kc = torch.full((B, Hkv, cap, D), canary, dtype=torch.float16, device="cuda")
+        return kc, kc.clone(), torch.zeros((B, H, D), dtype=torch.float32, device="cuda")
+
+    whole, parts, dx = buffers(), buffers(), dev(x)
+    with _ctx(H, Hkv, cap, B) as ctx:
+        ctx.qkv_append(dx, wq.w, wk.w, wv.w, whole[2], whole[0], whole[1], pos_tensor(pos), B)
+        assert ctx.device_status() == nw.NWD_ERR_DEVICE
+        assert ctx.device_status() == nw.NWD_OK
+    roomy_cap = 512  # a workspace for all rows; its caches' first rows are compared
+    with _ctx(H, Hkv, roomy_cap, B) as roomy:
+        for b in range(0, B, per):
+            m = min(per, B - b)
+            kc = torch.full((m, Hkv, roomy_cap, D), canary, dtype=torch.float16, device="cuda")
+            vc = kc.clone()
+            p = pos_tensor([v if v < cap else roomy_cap for v in pos[b:b + m]])
+            roomy.qkv_append(dx[b:b + m], wq.w, wk.w, wv.w, parts[2][b:b + m], kc, vc, p, m)
+            roomy.device_status()
+            parts[0][b:b + m], parts[1][b:b + m] = kc[:, :, :cap], vc[:, :, :cap]
+    for a, b in zip(whole, parts):
+        np.testing.assert_array_equal(host(a), host(b))
+    y64, bound = wq.f64(x)
+    assert np.all(np.abs(host(whole[2]).reshape(B, -1) - y64) <= TOL_REL * bound)
+    written = np.zeros((B, cap), bool)
+    for b in range(B):
+        if pos[b] < cap:
+            written[b, pos[b]] = True
+    for c in whole[:2]:
+        at = host(c) != np.float16(canary)
+        assert np.array_equal(at.any(axis=(1, 3)), written)
+
+
+@pytest.mark.parametrize("n,nb,rows,heads,per,records", [
+    (16384, 104, 48, 4, 32, lambda r: 256 if r <= 8 else 256 // -(-r // 16)),  # wide picks: 32 and 16 rows
+    (8192, 256, 50, 5, 16, lambda r: 512),                                     # the other kernel's
+])
+def test_lm_head_rows_in_small_workspace(n, nb, rows, heads, per, records):
+    say(f"lm_head rows in a small workspace n={n} n_blocks={nb} rows={rows}")
+    # past 32 rows both go to the kernel of one record per 32 (here 16) columns
+    many = 512 if n >= 16384 else 256
+    assert _launch_rows(nb, rows, _workspace(heads, heads, 16, 1),
+                        lambda r: records(r) if r <= 32 else many) == per
+    g = rng(956)
+    w = Q4(g, n, nb)
+    x = g.standard_normal((rows, 32 * nb)).astype(np.float32)
+    x[33, 7] = 1e9  # a wide row in the second launch
+    dx = dev(x)
+    logits = torch.full((rows, n), float("nan"), dtype=torch.float32, device="cuda")
+    parts = torch.empty_like(logits)
+    token = torch.full((2, rows), -1, dtype=torch.int32, device="cuda")
+    with _ctx(heads, heads, 16, 1) as ctx, _ctx() as roomy:
+        ctx.lm_head_argmax(dx, w.w, token[0], logits, rows)
+        for b in range(0, rows, per):
+            m = min(per, rows - b)
+            roomy.lm_head_argmax(dx[b:b + m], w.w, token[1, b:b + m], parts[b:b + m], m)
+        got, tok = host(logits), host(token)
+    np.testing.assert_array_equal(got, host(parts))
+    np.testing.assert_array_equal(tok[0], np.argmax(got, axis=1))
+    np.testing.assert_array_equal(tok[1], tok[0])
+    y64, bound = w.f64(x)
+    assert np.all(np.abs(got - y64) <= TOL_REL * bound)
+
+
+@pytest.mark.parametrize("n,nb,rows", [(20480, 98, 5), (20480, 33, 17), (4096, 98, 30)])
+def test_lm_head_rows_ties_and_non_finite(n, nb, rows):
+    """Logits that tie (columns repeated), rows of NaN and of one value: the
+    reference's tie order on every kernel."""
+    say(f"lm_head rows: ties, NaN n={n} n_blocks={nb} rows={rows}")
+    g = rng(957)
+    quant, scales, zp = random_q4(g, n // 256, nb)
+    cells = n // 256 * nb
+    z = np.stack([zp & 15, zp >> 4], axis=1).reshape(-1)[:cells].reshape(n // 256, nb)
+    quant, scales, z = (np.tile(a, (256,) + (1,) * (a.ndim - 1)) for a in (quant, scales, z))
+    z = z.reshape(-1, 2)
+    t = [dev(a) for a in (quant, scales, z[:, 0] | z[:, 1] << 4)]
+    w = nw.q4_weight(*t, n, nb)
+    x = g.standard_normal((rows, 32 * nb)).astype(np.float32)
+    x[1, 40] = np.nan
+    x[2, 3] = np.inf
+    x[3] = 0
+    x[4, 9] = 1e12  # a wide row
+    logits = torch.empty((rows, n), dtype=torch.float32, device="cuda")
+    token = torch.full((rows,), -1, dtype=torch.int32, device="cuda")
+    with _ctx() as ctx:
+        ctx.lm_head_argmax(dev(x), w, token, logits, rows)
+    got, tok = host(logits), host(token)
+    assert np.all(np.isnan(got[1:3])) and np.all(got[3] == 0)
+    for b in range(rows):
+        assert tok[b] == reference_rule(got[b]), b
+        if b not in (1, 2):
+            assert (got[b] == got[b].max()).sum() >= 256
 
 
 def test_rows_ranges_and_non_finite():
@@ -264,7 +403,7 @@ def test_qkv_rows(H, Hkv, q, Dh, B):
 
 @pytest.mark.parametrize("n,n_blocks,rows", [(20011, 98, 4), (20011, 98, 16), (16384, 97, 20), (33000, 33, 70),
                                                 (33001, 104, 48), (20017, 104, 48), (17001, 8, 48),
-                                                (20480, 105, 9)])
+                                                (20480, 105, 9), (16401, 130, 25), (16400, 160, 32)])
 def test_lm_head_rows(n, n_blocks, rows):
     say(f"lm_head rows n={n} n_blocks={n_blocks} rows={rows}")
     g = rng(970 + rows)
