@@ -30,8 +30,8 @@
 // multiplies. A workgroup of the latter stages the weights of 16 or 32
 // columns, all of K, in LDS with copies of whole runs of a column (reading 4
 // blocks at a time straight into the MFMA's lane order touched 3 cache lines
-// for 84 useful bytes of a column and took twice as long), its 8 wavefronts
-// split K and read the A operands of their part from L2.
+// for 84 useful bytes of a column and took twice as long), its 8 or 4
+// wavefronts split K and read the A operands of their part from L2.
 #include "nwd_argmax.h"
 #include "nwd_common.h"
 #include "nwd_internal.h"
@@ -352,7 +352,7 @@ __device__ inline void wide_sums(const RowsArgs& p, uint64_t wide, int row0, int
 
 // A workgroup owns kCols tiles of 16 columns, whose weights, all of K, it
 // stages in LDS at once, and walks row groups of kTiles row tiles (0:
-// packed). Its 8 wavefronts split the blocks of K.
+// packed). Its wavefronts split the blocks of K.
 // LDS of a 16-column tile, in cells (column, block): columns at an odd
 // stride, so that the 16 columns' reads of one block fall on distinct banks.
 __host__ __device__ inline int tile_cells(int n_blocks) { return 16 * (n_blocks | 1); }
@@ -551,17 +551,17 @@ __global__ __launch_bounds__(kWaves * 64, kTiles == 4 ? 2 : 4) void q4_product_k
 
 // ------------------------------------------------------- wide greedy picks
 
-// lm_head with the pick (pick_wide says which): one persistent workgroup per CU. Its
-// 8 wavefronts split K and hold their part of one row tile's A operands in
-// registers for the whole launch (read per 32 columns, as above, they were
+// lm_head with the pick (pick_wide says which): one persistent workgroup per
+// CU. Its 8 wavefronts split K and hold their part of one row tile's A operands
+// in registers for the whole launch (read per 32 columns, as above, they were
 // more L2 traffic than the weights); the weights of the next 32 columns, one
 // run of memory, lie in the other LDS buffer and those after it are on their
-// way in registers. Row tiles share the workgroups out, side
-// by side over the same columns, so that L2 and the Infinity Cache serve the
-// weights' second reading. A thread keeps the best of its logits of a row;
-// one record per row and workgroup. 131072 x 3136, us per call against the
-// kernel above: 4 rows 88 to 72, 16 rows 120 to 81, 32 rows 218 to 142. Its
-// products alone take 44 of them, its reads 55 (4.8 TB/s).
+// way in registers. Row tiles share the workgroups out, side by side over the
+// same columns, so that L2 and the Infinity Cache serve the weights' second
+// reading. A thread keeps the best of its logits of a row; one record per row
+// and workgroup. 131072 x 3136, us per call, the kernel above against this: 4
+// rows 98 against 68, 16 rows 118 against 75, 32 rows 171 against 135. Its
+// products alone take 44 of the 75, its reads 55 (4.8 TB/s).
 constexpr int kPickWaves = 8;
 constexpr int kPickThreads = kPickWaves * 64;
 constexpr int kPickCols = 32;
@@ -836,14 +836,15 @@ struct RowsPlan {
 
 // Row tiles: as few as hold the rows, up to 4 (64 rows: a wavefront's sums,
 // operands and products then fill its 256 registers). Two column tiles halve
-// what a workgroup reads of the A operands per column, which L2 bounds: for
-// wide projections, which fill the chip many times over, and with 4 row
-// tiles where the workgroups still fill half of it. us per call, one tile
-// against two: K = 3136, 64 rows, 7168 columns 27.1 against 19.8; 131072
-// columns, 4 and 16 rows 88.5 against 76.2 and 115 against 108; but K =
-// 3136, 16 and 32 rows, 7168 columns 12.6 against 12.9 and 15.3 against
-// 16.2, K = 5120, 16 and 64 rows, 3136 columns 11.4 against 14.2 and 22.4
-// against 24.2.
+// what a workgroup reads of the A operands per column, which L2 bounds with 4
+// row tiles, where the workgroups still fill half the chip: us per call, one
+// tile against two, K = 3136, 64 rows, 7168 columns 27.1 against 19.8. With fewer row
+// tiles two workgroups of one column tile to a CU overlap better, unless K is
+// short and each has little to do: 131072 columns, K = 256, 8 and 32 rows 52.4
+// against 40.8 and 55.5 against 51.1; K = 896 53.7 against 45.9 and 67.8
+// against 61.1; but K = 2048 71.5 against 70.2 and 132.5 against 167.9, K =
+// 3136, 16 rows 114.7 against 123.9, K = 4096, 8 rows 117.4 against 142.7,
+// and at 16384 columns K = 256, 16 rows 10.3 against 10.9.
 // Wavefronts: 8, or 4 where two such workgroups of 64 rows then fit a CU (by
 // their LDS) and the launch has them: 512 rows, K = 3136, 5120 columns 66.5
 // against 76.6; one workgroup per CU loses with 4 (K = 5120, 3136 columns
@@ -854,14 +855,15 @@ struct RowsPlan {
 // columns 76.6 / 80.0 / 99.2 us; K = 5120, 3136 columns 90.5 / 82.5 / 76.1;
 // K = 3136, 1024 columns 25.0 / 34.9 / 55.8.
 RowsPlan rows_plan(int cols, int n_blocks, int rows) {
-  constexpr int kCus = 256, kWide = 16384;
+  constexpr int kCus = 256, kWide = 32768, kShort = 48;
   RowsPlan r;
   r.tiles = rows <= kPackedRows ? 0 : (rows <= 16 ? 1 : (rows <= 32 ? 2 : 4));
   const int per = r.tiles ? 16 * r.tiles : kPackedRows, groups = (rows + per - 1) / per;
   const int64_t pairs = (cols + 31) / 32;
-  r.cols = n_blocks <= 160 && (cols >= kWide || (r.tiles == 4 && pairs * groups >= kCus / 2)) ? 2 : 1;
+  const bool two = r.tiles == 4 ? n_blocks <= 160 && pairs * groups >= kCus / 2 : n_blocks <= kShort && cols >= kWide;
+  r.cols = two ? 2 : 1;
   const int64_t wgs = r.cols == 2 ? pairs : (cols + 15) / 16;
-  r.waves = r.tiles == 4 && n_blocks <= 100 && wgs * groups >= 2 * kCus ? 4 : 8;
+  r.waves = r.cols == 2 && r.tiles == 4 && n_blocks <= 100 && wgs * groups >= 2 * kCus ? 4 : 8;
   const int64_t slots = r.waves == 4 ? 2 * kCus : kCus;
   r.split = 1;
   double best = 0;
@@ -880,11 +882,10 @@ RowsPlan rows_plan(int cols, int n_blocks, int rows) {
 // further row tile has it read and unpack the weights again: past 32 rows it
 // wins only near its longest K, where the other kernel's 64-row form has one
 // workgroup per CU, and with many columns. 131072 columns, the other kernel
-// against this, us: K = 3136, 16 rows 125 against 75, 32 rows 197 against 135,
+// against this, us: K = 3136, 16 rows 118 against 75, 32 rows 171 against 135,
 // 48 rows 203 against 195, 64 rows 211 against 252; K = 3328, 48 rows 241
-// against 202; K = 2560, 32 rows 179 against 119, 48 rows 168 against 170; K =
-// 896, 32 rows 93 against 79, 48 rows 96 against 113; 32768 columns, K = 3136,
-// 48 rows 62 against 63.
+// against 202; K = 2560, 48 rows 168 against 170; K = 896, 32 rows 93 against
+// 79, 48 rows 96 against 113; 32768 columns, K = 3136, 48 rows 62 against 63.
 constexpr int kPickGrid = 256;
 bool pick_wide(int cols, int n_blocks, int rows) {
   return cols >= 16384 && n_blocks <= kPickMaxBlocks &&
@@ -998,7 +999,7 @@ hipError_t launch_rows(RowsArgs p, const float* x, Q4Scratch scratch, uint32_t* 
   }
   NWD_ROWS_CASE(0, 1, 8) NWD_ROWS_CASE(0, 2, 8) NWD_ROWS_CASE(1, 1, 8) NWD_ROWS_CASE(1, 2, 8)
   NWD_ROWS_CASE(2, 1, 8) NWD_ROWS_CASE(2, 2, 8) NWD_ROWS_CASE(4, 1, 8) NWD_ROWS_CASE(4, 2, 8)
-  NWD_ROWS_CASE(4, 1, 4) NWD_ROWS_CASE(4, 2, 4)
+  NWD_ROWS_CASE(4, 2, 4)
 #undef NWD_ROWS_CASE
   return hipErrorInvalidValue;
 }
@@ -1022,17 +1023,17 @@ RowsArgs rows_args(const Q4Mat* m, int n_mats, int n_blocks) {
 // 8192, 64 columns, 96 rows 9.5 against 31.6, 512 columns, 17 rows 13.5
 // against 18.8, 2048 columns, 3 rows 11.3 against 12.5; K = 3136, 256
 // columns, 64 rows 10.3 against 16.6; K = 5120, 100 columns, 96 rows 12.0
-// against 24.2, 16 columns, 4000 rows 60 against 129; with the pick, K = 4096,
-// 131072 columns, 2 rows 121 against 149 and K = 896 31 against 43. Over K of 32
-// to 8192, 16 to 16384 columns and 2 to 4000 rows (picks: 4096 to 131072 columns, 2 to 64 rows),
-// 2000 shapes past the bound of q4_rows_shape, the choice lost more than 6%
-// against the one-row kernels at one (12%: K = 8192, 48 columns, 2000 rows)
-// and more than 13% against the matrix cores at one (18%: K = 8192, 100
+// against 24.2, 16 columns, 4000 rows 60 against 129; with the pick, 131072
+// columns, 2 rows, K = 896 31 against 43, K = 2048 56 against 59. Over K of 32 to
+// 8192, 16 to 131072 columns and 2 to 4000 rows (picks: 4096 columns up, 2 to
+// 64 rows), 2100 shapes past the bound of q4_rows_shape, the choice lost more
+// than 7% against the one-row kernels at one (14%: K = 8192, 48 columns, 2000
+// rows) and more than 13% against the matrix cores at one (18%: K = 8192, 100
 // columns, 256 rows).
 double one_row_us(int cols, int n_blocks, int rows, bool pick) {
   const double nb = n_blocks;
   // lm_head's form (128-thread workgroups, K in registers), per column and row
-  if (pick && cols >= 16384) return 8 + 1e-3 * rows * cols * (0.03 + (0.0016 + 0.0000125 * nb) * nb);
+  if (pick && cols >= 16384) return 8 + 1e-3 * rows * cols * (0.03 + (0.0016 + 0.0000118 * nb) * nb);
   // per 16 columns and row, by the wavefronts that share K (q4_split)
   const double unit = nb < 64 ? 1.8 + 0.038 * nb : (nb < 128 ? 2.6 + 0.0475 * nb : 4.8 + 0.052 * nb);
   return (pick ? 8 : 3) + 1e-3 * rows * ((cols + 15) / 16) * unit;
@@ -1041,15 +1042,16 @@ double several_rows_us(int cols, int n_blocks, int rows, bool pick) {
   const double nb = n_blocks;
   if (pick && pick_wide(cols, n_blocks, rows)) return 11.5 + 1e-3 * pick_tiles(rows) * cols * (0.15 + 0.0036 * nb);
   const RowsPlan p = rows_plan(cols, n_blocks, rows);
-  // a row group's time per block of K, by row tiles (packed, 1, 2, 4) and column tiles
-  constexpr double kGroup[2][4] = {{0.019, 0.025, 0.046, 0.092}, {0.059, 0.073, 0.109, 0.124}};
+  // a round of workgroups, and its row groups' time per block of K, by row
+  // tiles (packed, 1, 2, 4) and column tiles
+  constexpr double kRound[2] = {0.9, 1.9}, kGroup[2][4] = {{0.0195, 0.026, 0.046, 0.092}, {0.017, 0.025, 0.046, 0.114}};
   const int wg_rows = p.tiles ? 16 * p.tiles : kPackedRows, groups = (rows + wg_rows - 1) / wg_rows;
   const int64_t wgs = (cols + 16 * p.cols - 1) / (16 * p.cols) * (int64_t)p.split;
   const int64_t slots = p.waves == 4 ? 512 : 256, rounds = (wgs + slots - 1) / slots;
   const double operands = 1e-3 * rows * nb;  // written and read once, past L2 where many
-  return (pick ? 10 : 7) + (0.1 + 0.0001 * operands) * operands +
-         kGroup[p.cols - 1][p.tiles == 4 ? 3 : p.tiles] * nb * rounds * ((groups + p.split - 1) / p.split) *
-             (p.waves == 4 ? 2 : 1);
+  return (pick ? 10 : 6) + (0.1 + 0.0001 * operands) * operands +
+         rounds * (kRound[p.cols - 1] + kGroup[p.cols - 1][p.tiles == 4 ? 3 : p.tiles] * nb *
+                                            ((groups + p.split - 1) / p.split) * (p.waves == 4 ? 2 : 1));
 }
 
 }  // namespace

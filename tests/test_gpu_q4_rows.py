@@ -68,7 +68,8 @@ def _ctx(H=32, Hkv=8, cap=512, B=64, q="f32", Dh=D):
     (520, 256, 130),   # the largest K
     (48, 1, 40000),    # one block: most wavefronts have none
     (777, 5, 500),
-    (16400, 40, 8), (16400, 40, 16), (16400, 40, 32),  # two column tiles: wide projections
+    (32790, 40, 8), (32790, 40, 16), (32790, 40, 32),  # two column tiles: wide, of short K
+    (16400, 98, 8), (16400, 98, 20),                   # and of long K: one
 ])
 def test_rows_match_float64(n, n_blocks, rows):
     say(f"q4 rows n={n} n_blocks={n_blocks} rows={rows}")
