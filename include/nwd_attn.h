@@ -317,13 +317,19 @@ enum {
  * y[b][n] = epilogue(W . a[b]). a is [batch][32 * n_blocks] f32 (16-byte
  * aligned), y [batch][n] f32. Dispatched as ceil(N / 4) workgroups by the
  * reference (engine/runtime.js:359-361); here the library picks the grid.
- * Calls of several rows (and nwd_qkv_append's, nwd_lm_head_argmax's) past a
- * size run on fp16 MFMAs, the activations carried as high and low parts in
- * the context's workspace: closer to 64 bits than the one-row kernels. */
+ * Calls of several rows (and nwd_qkv_append's, nwd_lm_head_argmax's) run on
+ * fp16 MFMAs where those are faster, the activations carried as high and low
+ * parts in the context's workspace, each within 2^-23 of the largest of its
+ * 32, or in fp32 in rows whose range is too wide for that: closer to 64 bits
+ * than the one-row kernels. A row's sums are then taken in an order that
+ * depends on the number of rows, so its results may differ in rounding
+ * between batch sizes (and a greedy pick between logits that nearly tie);
+ * equal calls give equal bits. */
 int nwd_q4_gemv(nwd_ctx* ctx, const float* a, const nwd_q4_weight* w, float* y,
                 int32_t batch, int32_t epilogue, void* stream);
 
-/* The attention layer's q / k / v projections and kv_append in one launch:
+/* The attention layer's q / k / v projections and kv_append in one launch
+ * (several rows: two, one of them converting x):
  * the dispatches L-q, L-k, L-v, L-kvK and L-kvV of engine/runtime.js:386-390
  * (matmul_nbits_sg.wgsl three times, then kv_append.wgsl:12-18 for k and
  * v). x is [batch][K] f32 (the normalised hidden state, 16-byte aligned); wq
