@@ -22,16 +22,18 @@
 // row's (an activation of 10^6 beside ordinary ones) would lose bits there
 // that a weight of zero at the large element brings to light: such a row is
 // "wide", and its sums are taken in fp32 from the activations themselves, by
-// the same wavefronts over the weights in LDS (wide_dot). So every x is held
-// within 2^-23 of the largest magnitude of its block, at least.
+// the same wavefronts over the weights in LDS (wide_sums) or by a wide pick's
+// merge. So every x is held within 2^-23 of the largest magnitude of its
+// block, at least.
 //
 // Two launches per call: q4_rows_kernel converts the activation rows into
 // the A operands' lane order in the context's workspace, q4_product_kernel
-// multiplies. A workgroup of the latter stages the weights of 16 or 32
-// columns, all of K, in LDS with copies of whole runs of a column (reading 4
-// blocks at a time straight into the MFMA's lane order touched 3 cache lines
-// for 84 useful bytes of a column and took twice as long), its 8 or 4
-// wavefronts split K and read the A operands of their part from L2.
+// multiplies; picks add the merge of their records. A workgroup of the product
+// kernel stages the weights of 16 or 32 columns, all of K, in LDS with copies
+// of whole runs of a column (reading 4 blocks at a time straight into the
+// MFMA's lane order touched 3 cache lines for 84 useful bytes of a column and
+// took twice as long), its 8 or 4 wavefronts split K and read the A operands
+// of their part from L2.
 #include "nwd_argmax.h"
 #include "nwd_common.h"
 #include "nwd_internal.h"
@@ -43,7 +45,7 @@ namespace nwd {
 namespace {
 
 // Cells (columns) of up to three projections side by side, the argument block
-// of both kernels.
+// of the kernels.
 struct RowsArgs {
   Q4Mat m[3];
   int n_mats;

@@ -466,3 +466,42 @@ def test_lm_head_fills_the_workspace():
             assert np.all(np.abs(got[0] - y64[:rows]) <= TOL_REL * bound[:rows])
         with pytest.raises(nw.NwdError):
             small.lm_head_argmax(dx, w.w, torch.empty(129, dtype=torch.int32, device="cuda"), None, 129)
+
+
+def test_rows_in_a_graph():
+    """q/k/v, a projection onto it and the wide pick of several rows, captured
+    once and replayed on new activations (wide rows in some), with eager calls
+    between: every replay gives the eager bits."""
+    say("q4 rows in a graph")
+    H, Hkv, cap, B, nb = 8, 8, 16, 12, 98
+    g = rng(995)
+    wq, wk, wv = Q4(g, H * D, nb), Q4(g, Hkv * D, nb), Q4(g, Hkv * D, nb)
+    wo, wl = Q4(g, 4096, H * D // 32), Q4(g, 16390, nb)
+    x = torch.zeros((B, 32 * nb), dtype=torch.float32, device="cuda")
+    pos = pos_tensor([b % cap for b in range(B)])
+
+    def buffers():
+        kc = torch.zeros((B, Hkv, cap, D), dtype=torch.float16, device="cuda")
+        return (torch.zeros((B, H * D), device="cuda"), kc, kc.clone(), torch.zeros((B, 4096), device="cuda"),
+                torch.zeros((B, 16390), device="cuda"), torch.zeros(B, dtype=torch.int32, device="cuda"))
+
+    def run(ctx, stream, q, kc, vc, h, logits, token):
+        ctx.qkv_append(x, wq.w, wk.w, wv.w, q, kc, vc, pos, B, stream=stream)
+        ctx.q4_gemv(q, wo.w, h, B, stream=stream)
+        ctx.lm_head_argmax(x, wl.w, token, logits, B, stream=stream)
+
+    captured, eager = buffers(), buffers()
+    with _ctx(H, Hkv, cap, B) as ctx, _ctx(H, Hkv, cap, B) as other:
+        stream = torch.cuda.Stream()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            run(ctx, stream, *captured)
+        for i in range(4):
+            v = g.standard_normal((B, 32 * nb)).astype(np.float32)
+            if i % 2:
+                v[i, 9] = 1e12
+            x.copy_(dev(v))
+            graph.replay()
+            run(other, None, *eager)
+            for a, b in zip(captured, eager):
+                np.testing.assert_array_equal(host(a), host(b))
