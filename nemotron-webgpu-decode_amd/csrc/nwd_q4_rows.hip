@@ -930,7 +930,8 @@ RowsLayout rows_layout(int cols, int n_blocks, int rows, bool pick) {
 int rows_per_launch(int cols, int n_blocks, int rows, bool pick, size_t scratch) {
   const auto fits = [&](int r) { return rows_layout(cols, n_blocks, r, pick).bytes <= scratch; };
   if (fits(rows)) return rows;
-  for (int r = (rows - 1) / 64 * 64; r >= 64; r -= 64)
+  const size_t operands = scratch / ((size_t)n_blocks * 128);  // rows whose operands alone fit
+  for (int r = (operands < (size_t)rows ? (int)operands : rows - 1) / 64 * 64; r >= 64; r -= 64)
     if (fits(r)) return r;
   for (int r : {32, 16, kPackedRows})
     if (r < rows && fits(r)) return r;
